@@ -250,10 +250,9 @@ int n3ds_render_extras(const float* state, const float* tdist, const float* dire
  * gradient groups queued per SDF family across rays (0..1, default 1), 5 = the
  * culling pass of one scene with the stroke grid (0..1, default 1), 6 = the
  * split adjoint when its workspace is given (0..1, default 1), 7 = records per
- * ray and SDF family the split adjoint's lists hold (1..1024, default 32; a
- * fuller list sends every ray to the one-kernel adjoint).  value < 0 only
- * queries.  Returns the previous
- * value, or -1 for an unknown parameter or a value out of range.  Results do
+ * ray and SDF family the split adjoint's pool is sized for (1..1024, default 32;
+ * rays that find the pool empty are left to the one-kernel adjoint).  value < 0
+ * only queries.  Returns the previous value, or -1 for an unknown parameter or a value out of range.  Results do
  * not depend on these parameters beyond float summation order. */
 int n3ds_render_tuning(int param, int value);
 
@@ -273,7 +272,8 @@ int64_t n3ds_render_backward_workspace_floats(int64_t n_rays, int n_strokes, int
  * adjoint as a per-ray kernel that lists the live (sample, stroke) pairs' adjoint
  * records per SDF family and a kernel over those records, when its workspace holds
  * max(this, n3ds_render_backward_workspace_floats(...)) floats; same results up to
- * the float summation order of the gradients. */
+ * the float summation order of the gradients.  A larger workspace holds more
+ * records (8 floats each), for scenes with many live pairs per ray. */
 int64_t n3ds_render_backward_split_floats(int64_t n_rays, int n_strokes, int shape_width, int color_width);
 
 /* Backward: accumulates dL/d(shape_params) [S,shape_width], dL/d(color_params)

@@ -33,6 +33,7 @@
 // Sample depths must be non-decreasing along a ray (as the reference's
 // stratified samplers produce); a ray whose depths are not sorted falls back
 // to evaluating every hit stroke on all its samples (same result, slower).
+#include <algorithm>
 #include <mutex>
 
 #include "n3ds_capi.h"
@@ -111,19 +112,19 @@ struct RenderArgs {
     int64_t ntask;    // culling tasks: rays x chunk groups (a batch: each scene's own chunks)
     int cull_group;   // chunks culled by one culling task
     int flush_pairs;  // pending pairs that trigger evaluation
-    // split adjoint (render_bwd_kernel MODE 2, then render_bwd_pairs_kernel): per SDF
-    // family and MODE 2 wavefront a field-major region of sp_cap adjoint records
-    // (stroke, ray, depth, dL/dalpha, dL/d(density), dL/d(colour) x 3), sp_count [NCLASS,
-    // sp_nw] the 64-record groups each region holds (then their exclusive prefix and the
-    // total, group_scan_kernel), sp_ovf set when a region overflowed
-    // (the fused kernel then takes every ray), fbflag [R] the rays left to the fused
-    // kernel; nullptr outside the split adjoint
+    // split adjoint (render_bwd_kernel MODE 2, then render_bwd_pairs_kernel): sp_list is a
+    // pool of sp_pages pages of SP_PAGE adjoint records of one SDF family, field-major
+    // (stroke, ray, depth, dL/dalpha, dL/d(density), dL/d(colour) x 3); the first
+    // sp_first pages are the MODE 2 wavefronts' own, sp_next counts the pages asked for
+    // beyond them (past sp_pages: the pool ran out), sp_count [sp_pages + 1] the
+    // 64-record groups of each page (then their exclusive prefix and the total,
+    // page_scan_kernel), fbflag [R] the rays left to the fused kernel; nullptr outside the
+    // split adjoint
     float* sp_list;
     int* sp_count;
-    int* sp_ovf;
+    int* sp_next;
     int* fbflag;
-    int64_t sp_cap;
-    int sp_nw;
+    int sp_pages, sp_first;
 };
 
 constexpr int SCENE_REC = 10;
@@ -2366,38 +2367,63 @@ __device__ __forceinline__ void queued_group(const RenderArgs& A, const WaveMem&
 
 __host__ __device__ constexpr int pairs_wave_floats(int ng) { return 64 * (ng + 1) + 64; }
 
-// One block: c[0..n) (group counts) replaced by their exclusive prefix, the total in c[n];
-// also clears z[0..nz).
-__global__ __launch_bounds__(1024) void group_scan_kernel(int* __restrict__ c, int64_t n, float* __restrict__ z,
-                                                          int64_t nz) {
-    __shared__ int part[1024];
-    const int t = threadIdx.x;
-    for (int64_t i = t; i < nz; i += 1024) z[i] = 0.f;
-    const int64_t per = (n + 1023) / 1024, b0 = min((int64_t)t * per, n), b1 = min(b0 + per, n);
-    int sum = 0;
-    for (int64_t i = b0; i < b1; i++) sum += c[i];
-    part[t] = sum;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {  // inclusive scan of the per-thread sums
-        const int v = t >= off ? part[t - off] : 0;
+// Records per page of the split adjoint's pool.  A wavefront starts with one open page per
+// SDF family and takes further ones from a device-wide counter, one returning atomic per
+// SP_PAGE records (a counter bumped by every window made the per-ray kernel markedly slower).  A
+// window holds at most PBUF pairs, so one new page always takes what the open one cannot.
+// Sharing the pool matters: with a fixed region per wavefront, one wavefront whose rays
+// run along dense strokes overflowed and sent every ray to the fused kernel (854 us of the
+// 1.80 ms step at 500 strokes x 65536 rays x 128 samples; the pool holds 2.5x that
+// workload's records).
+constexpr int SP_PAGE = 256;
+static_assert(SP_PAGE >= PBUF && SP_PAGE % 64 == 0, "a window fits one new page");
+
+// One block: the group counts of the pages handed out replaced by their exclusive prefix,
+// the total behind the last; also clears z[0..nz).  Tiles of 4096 counts, four per thread:
+// wavefront scans by shuffles, the 16 wavefront totals through LDS.
+constexpr int SCAN_THREADS = 1024;
+__global__ __launch_bounds__(SCAN_THREADS) void page_scan_kernel(int* __restrict__ c, const int* __restrict__ next,
+                                                                 int first, int pages, float* __restrict__ z,
+                                                                 int64_t nz) {
+    __shared__ int wtot[SCAN_THREADS / 64];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    for (int64_t i = t; i < nz; i += SCAN_THREADS) z[i] = 0.f;
+    const int n = min(first + *next, pages);
+    int carry = 0;
+    for (int b0 = 0; b0 < n; b0 += 4 * SCAN_THREADS) {
+        const int i0 = b0 + 4 * t;
+        int v[4], sum = 0;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            v[q] = i0 + q < n ? c[i0 + q] : 0;
+            sum += v[q];
+        }
+        const int incl = wave_incl_scan(sum, lane);
+        if (lane == 63) wtot[wave] = incl;
         __syncthreads();
-        part[t] += v;
+        int before = 0, total = 0;
+#pragma unroll
+        for (int q = 0; q < SCAN_THREADS / 64; q++) {
+            if (q < wave) before += wtot[q];
+            total += wtot[q];
+        }
+        int run = carry + before + incl - sum;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            if (i0 + q < n) c[i0 + q] = run;
+            run += v[q];
+        }
+        carry += total;
         __syncthreads();
     }
-    int run = part[t] - sum;
-    for (int64_t i = b0; i < b1; i++) {
-        const int v = c[i];
-        c[i] = run;
-        run += v;
-    }
-    if (t == 1023) c[n] = part[1023];
+    if (t == 0) c[n] = carry;
 }
 constexpr int PAIRS_WAVES = 16;  // wavefronts per block of the pair kernel at most (one block per CU)
 
 // Split adjoint, second kernel: the records of render_bwd_kernel<MODE 2>, 64 of one SDF
 // family per wavefront, through pair_grad; each stroke's run of lanes is summed into the
-// block's rows (LDS, or the global rows) as in the fused kernel.  Does nothing when a
-// region overflowed (the fused kernel then takes every ray).
+// block's rows (LDS, or the global rows) as in the fused kernel.  When the pool ran out,
+// records of a ray that is flagged for the fused kernel are skipped.
 template <int CID>
 __global__ __launch_bounds__(64 * PAIRS_WAVES) void render_bwd_pairs_kernel(RenderArgs A, float* __restrict__ partials,
                                                                        int use_lds, float* __restrict__ gdirect) {
@@ -2413,42 +2439,44 @@ __global__ __launch_bounds__(64 * PAIRS_WAVES) void render_bwd_pairs_kernel(Rend
     WaveMem w;
     w.scr = smem + nacc + (int64_t)wave * pairs_wave_floats(NG);
     w.xo = (int*)(w.scr + 64 * (NG + 1));
-    // sp_count holds, after grid_scan_kernel, the groups before each region (and the total
-    // at index nreg); wavefront q takes groups [q G / Q, (q + 1) G / Q)
-    const int64_t nreg = (int64_t)NCLASS * A.sp_nw;
-    const int64_t total = *A.sp_ovf == 0 ? A.sp_count[nreg] : 0;
+    // sp_count holds, after page_scan_kernel, the groups before each page (and the total
+    // behind the last); wavefront q takes groups [q G / Q, (q + 1) G / Q)
+    const int asked = A.sp_first + *A.sp_next;
+    const int npg = min(asked, A.sp_pages);
+    const bool lost = asked > A.sp_pages;
+    const int64_t total = A.sp_count[npg];
     const int64_t nq = (int64_t)gridDim.x * W, q = (int64_t)blockIdx.x * W + wave;
     const int64_t g0 = total * q / nq, g1 = total * (q + 1) / nq;
-    int64_t rg = 0;
-    if (g0 < g1) {  // the region of group g0: the last one starting at or before it
-        int64_t lo = 0, hi = nreg - 1;
+    int pg = 0;
+    if (g0 < g1) {  // the page of group g0: the last one starting at or before it
+        int lo = 0, hi = npg - 1;
         while (lo < hi) {
-            const int64_t mid = (lo + hi + 1) >> 1;
+            const int mid = (lo + hi + 1) >> 1;
             if (A.sp_count[mid] <= g0) lo = mid;
             else hi = mid - 1;
         }
-        rg = lo;
+        pg = lo;
     }
     for (int64_t g = g0; g < g1; g++) {
-        while (A.sp_count[rg + 1] <= g) rg++;  // skip regions without groups
+        while (A.sp_count[pg + 1] <= g) pg++;  // skip pages without groups
         {
-            const int64_t gi = g - A.sp_count[rg];
-            const float* L = A.sp_list + rg * RW * A.sp_cap + gi * 64 + lane;
+            const int gi = (int)(g - A.sp_count[pg]);
+            const float* L = A.sp_list + (int64_t)pg * (RW * SP_PAGE) + gi * 64 + lane;
             const int k = __float_as_int(L[0]);
             float G[NG];
 #pragma unroll
             for (int q = 0; q < NG; q++) G[q] = 0.f;
-            if (k >= 0) {
-                const int64_t ray = __float_as_int(L[A.sp_cap]);
-                const float t = L[2 * A.sp_cap];
+            const int64_t ray = k >= 0 ? __float_as_int(L[SP_PAGE]) : 0;
+            if (k >= 0 && !(lost && A.fbflag[ray])) {
+                const float t = L[2 * SP_PAGE];
                 const V3 o = ld3(A.origins + 3 * ray), d = ld3(A.dirs + 3 * ray), vd = ld3(A.viewdirs + 3 * ray);
                 V3 x = d * t + o;
                 if (A.coord_div != 1.f) x = v3(x.x / A.coord_div, x.y / A.coord_div, x.z / A.coord_div);
                 const float r = A.cone ? A.radii[ray] * t : A.radii[ray];
-                pair_grad<CID>(A, k, x, r, vd, L[3 * A.sp_cap], L[4 * A.sp_cap],
-                               v3(L[5 * A.sp_cap], L[6 * A.sp_cap], L[7 * A.sp_cap]), G);
+                pair_grad<CID>(A, k, x, r, vd, L[3 * SP_PAGE], L[4 * SP_PAGE],
+                               v3(L[5 * SP_PAGE], L[6 * SP_PAGE], L[7 * SP_PAGE]), G);
             }
-            // empty records only pad a region's last group, so the valid lanes lead it
+            // empty records only pad a page's last group, so the valid lanes lead it
             const int nl = __popcll(__ballot(k >= 0));
             reduce_runs<NG>(A, w, lane, nl, k >= 0 ? k : 0x7fffffff, G, dst, PG);
         }
@@ -2462,11 +2490,10 @@ __global__ __launch_bounds__(64 * PAIRS_WAVES) void render_bwd_pairs_kernel(Rend
 
 // MODE 0: gradient groups window by window; 1: the pending-pair queues (queues !=
 // nullptr), full groups of one family across rays; 2: the first kernel of the split
-// adjoint: rays whose hits were all kept and fit the pending list append their live
-// pairs' records to this wavefront's region of each family list instead of evaluating
-// them (the last group padded with empty records), the other rays are flagged for the
-// fused kernel.  With fbflag set, MODE 1 takes only the flagged rays (every ray after
-// an overflow).
+// adjoint: rays whose hits were all kept append their live pairs' records to this
+// wavefront's open page of each family instead of evaluating them (a page's last group
+// padded with empty records); the other rays, and a ray that finds the pool empty, are
+// flagged for the fused kernel.  With fbflag set, MODE 1 takes only the flagged rays.
 template <int NS, int CID, int MODE>
 __global__ __launch_bounds__(64 * BWAVES) void render_bwd_kernel(RenderArgs A0, const float* __restrict__ g_rgb,
                                                                  const float* __restrict__ g_acc,
@@ -2511,15 +2538,14 @@ __global__ __launch_bounds__(64 * BWAVES) void render_bwd_kernel(RenderArgs A0, 
     __syncthreads();
     const WaveMem w = wave_mem(smem + nacc_max + wave * wave_mem_floats(NS, NPF, NGL), NS, NPF, NGL);
     const int64_t N = A.R * (int64_t)A.n;
-    const bool fb_all = MODE == 1 && A.fbflag && *A.sp_ovf != 0;
-    // MODE 2: this wavefront's list regions and how many records each holds
-    const int64_t wid = (int64_t)blockIdx.x * W + wave;
+    // MODE 2: this wavefront's open pages and how many records each holds
+    const int own = NCLASS * (int)(blockIdx.x * W + wave);
+    int page[NCLASS] = {own, own + 1, own + 2};
     int cur[NCLASS] = {0, 0, 0};
-    bool full = false;
     unsigned long long fmask = 0ull;  // MODE 1 with fbflag: flags of this wavefront's next 64 rays
     for (int64_t ray = ray0, it = 0; ray < ray_end; ray += ray_step, it++) {
         if constexpr (MODE == 1) {
-            if (A.fbflag && !fb_all) {  // rays done by the split adjoint are skipped
+            if (A.fbflag) {  // rays done by the split adjoint are skipped
                 if ((it & 63) == 0) {
                     const int64_t mine = ray + lane * ray_step;
                     fmask = __ballot(mine < ray_end && A.fbflag[mine] != 0);
@@ -2633,7 +2659,7 @@ __global__ __launch_bounds__(64 * BWAVES) void render_bwd_kernel(RenderArgs A0, 
         int d0 = -1, d1 = 0, d2 = 0;  // kept chunk records of chunks (ch & ~63) + lane
         // every chunk kept and the hits fit the pending list: gather them in one pass (a
         // ray's kept hits and pairs are contiguous from its first chunk's offsets)
-        bool preloaded = false;
+        bool preloaded = false, all_kept = false;
         if (A.hdir && A.nch <= 64) {
             if (lane < A.nch) {
                 const int* e = A.hdir + (ray * A.nch_stride + lane) * 3;
@@ -2641,7 +2667,7 @@ __global__ __launch_bounds__(64 * BWAVES) void render_bwd_kernel(RenderArgs A0, 
                 d1 = e[1];
                 d2 = e[2];
             }
-            const bool all_kept = __ballot(lane < A.nch && d0 < 0) == 0ull;
+            all_kept = __ballot(lane < A.nch && d0 < 0) == 0ull;
             int H = d2;
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) H += __shfl_xor(H, off, 64);
@@ -2669,7 +2695,7 @@ __global__ __launch_bounds__(64 * BWAVES) void render_bwd_kernel(RenderArgs A0, 
             }
         }
         if constexpr (MODE == 2) {
-            if (!preloaded) {  // left to the fused kernel
+            if (!all_kept) {  // left to the fused kernel
                 if (lane == 0) A.fbflag[ray] = 1;
                 continue;
             }
@@ -2874,26 +2900,48 @@ __global__ __launch_bounds__(64 * BWAVES) void render_bwd_kernel(RenderArgs A0, 
                 wave_sync();
                 const int nu = xs[NCLASS];
                 if constexpr (MODE == 2) {
-                    // append the live pairs class by class to this wavefront's regions
+                    // append the live pairs class by class to this wavefront's open pages
+                    bool lost = false;
 #pragma unroll
                     for (int xc = 0; xc < NCLASS; xc++) {
                         const int nx = xs[xc + 1] - xs[xc];
-                        if (cur[xc] + nx > A.sp_cap) full = true;
-                        if (full) continue;
-                        float* L = A.sp_list + ((int64_t)xc * A.sp_nw + wid) * RW * A.sp_cap + cur[xc];
+                        if (nx == 0 || lost) continue;
+                        int fresh = -1;
+                        if (cur[xc] + nx > SP_PAGE) {
+                            int got = 0;
+                            if (lane == 0) got = atomicAdd(A.sp_next, 1);
+                            fresh = A.sp_first + __builtin_amdgcn_readfirstlane(got);
+                            if (fresh >= A.sp_pages) {
+                                lost = true;
+                                continue;
+                            }
+                        }
                         for (int u = lane; u < nx; u += 64) {
                             const int e = w.ul[xs[xc] + u];
                             const int p = e & 0xffff, c = e >> 16;
-                            L[u] = __int_as_float(w.ck[c]);
-                            L[A.sp_cap + u] = __int_as_float((int)ray);
-                            L[2 * A.sp_cap + u] = w.ts[w.ci0[c] + (p - (w.coff[c] - wbase))];
-                            L[3 * A.sp_cap + u] = w.pb[p];
-                            L[4 * A.sp_cap + u] = w.pb[PBUF + p];
-                            L[5 * A.sp_cap + u] = w.pb[2 * PBUF + p];
-                            L[6 * A.sp_cap + u] = w.pb[3 * PBUF + p];
-                            L[7 * A.sp_cap + u] = w.pb[4 * PBUF + p];
+                            const int slot = cur[xc] + u;
+                            float* L = A.sp_list + (int64_t)(slot < SP_PAGE ? page[xc] : fresh) * (RW * SP_PAGE) +
+                                       slot % SP_PAGE;
+                            L[0] = __int_as_float(w.ck[c]);
+                            L[SP_PAGE] = __int_as_float((int)ray);
+                            L[2 * SP_PAGE] = w.ts[w.ci0[c] + (p - (w.coff[c] - wbase))];
+                            L[3 * SP_PAGE] = w.pb[p];
+                            L[4 * SP_PAGE] = w.pb[PBUF + p];
+                            L[5 * SP_PAGE] = w.pb[2 * PBUF + p];
+                            L[6 * SP_PAGE] = w.pb[3 * PBUF + p];
+                            L[7 * SP_PAGE] = w.pb[4 * PBUF + p];
                         }
                         cur[xc] += nx;
+                        if (fresh >= 0) {  // the page before is full
+                            if (lane == 0) A.sp_count[page[xc]] = SP_PAGE / 64;
+                            page[xc] = fresh;
+                            cur[xc] -= SP_PAGE;
+                        }
+                    }
+                    if (lost) {  // the pool is empty: the fused kernel takes this ray
+                        if (lane == 0) A.fbflag[ray] = 1;
+                        ch = A.nch;
+                        break;
                     }
                 } else if constexpr (QUEUE) {
                     // queue the live pairs class by class behind the pending ones; a class's
@@ -3026,15 +3074,14 @@ __global__ __launch_bounds__(64 * BWAVES) void render_bwd_kernel(RenderArgs A0, 
             nh = np = 0;
         }
     }
-    if constexpr (MODE == 2) {  // pad each region to whole groups; a full region sends every ray to MODE 1
+    if constexpr (MODE == 2) {  // pad each open page to whole groups
 #pragma unroll
         for (int xc = 0; xc < NCLASS; xc++) {
-            const int padded = (cur[xc] + 63) / 64 * 64;  // <= sp_cap, a multiple of 64
-            float* L = A.sp_list + ((int64_t)xc * A.sp_nw + wid) * RW * A.sp_cap;
-            if (!full && cur[xc] + lane < padded) L[cur[xc] + lane] = __int_as_float(-1);
-            if (lane == 0) A.sp_count[(int64_t)xc * A.sp_nw + wid] = full ? 0 : padded / 64;
+            const int padded = (cur[xc] + 63) / 64 * 64;
+            float* L = A.sp_list + (int64_t)page[xc] * (RW * SP_PAGE);
+            if (cur[xc] + lane < padded) L[cur[xc] + lane] = __int_as_float(-1);
+            if (lane == 0) A.sp_count[page[xc]] = padded / 64;
         }
-        if (full && lane == 0) *A.sp_ovf = 1;
     } else if constexpr (QUEUE) {  // the partial groups left in the queues
 #pragma unroll
         for (int xc = 0; xc < NCLASS; xc++)
@@ -3120,8 +3167,8 @@ static int g_max_lds = 0;
 // one scene tests only the strokes of its ray's grid cells (1) or every stroke (0).
 // TUNE_BWD_SPLIT: with kept hits, the adjoint runs as a per-ray kernel that lists the
 // live pairs' records and a kernel over the records (1), or as one kernel (0);
-// TUNE_SPLIT_CAP: list records per ray and SDF family (an overflow falls back to the one
-// kernel for every ray).
+// TUNE_SPLIT_CAP: list records per ray and SDF family the workspace is sized for (rays
+// past the pool fall back to the one kernel).
 enum {
     TUNE_FLUSH_PAIRS = 0, TUNE_BWD_OVERSUB = 1, TUNE_BATCH_OVERSUB = 2, TUNE_CULL_GROUP = 3, TUNE_BWD_QUEUE = 4,
     TUNE_CULL_GRID = 5, TUNE_BWD_SPLIT = 6, TUNE_SPLIT_CAP = 7, TUNE_COUNT = 8
@@ -3279,10 +3326,9 @@ static RenderArgs make_args(const float* origins, const float* dirs, const float
     A.ntask = 0;
     A.sp_list = nullptr;
     A.sp_count = nullptr;
-    A.sp_ovf = nullptr;
+    A.sp_next = nullptr;
     A.fbflag = nullptr;
-    A.sp_cap = 0;
-    A.sp_nw = 0;
+    A.sp_pages = A.sp_first = 0;
     return A;
 }
 
@@ -3507,7 +3553,8 @@ N3DS_EXPORT int n3ds_render_forward(const float* origins, const float* direction
 // Split adjoint launch plan: the per-ray kernel (MODE 2, SPLIT_WAVES wavefronts per
 // block, no gradient rows), the pair kernel and the fused kernel for flagged rays (both
 // with per-block gradient rows in LDS), and the workspace pieces in floats: gradient
-// rows of both, the two kernels' queues, the family lists, then the counters and flags.
+// rows of both, the fused kernel's queues, the page counter and ray flags, then the pages
+// with their group counts (as many as the workspace given holds, at least min_pages).
 constexpr int SPLIT_WAVES = 4;
 
 struct SplitPlan {
@@ -3517,9 +3564,12 @@ struct SplitPlan {
     int64_t lds1, lds2;
     int pw;  // wavefronts per block of the pair kernel
     BwdShape bsf;
-    int64_t cap;  // records per region (a multiple of 64)
-    int64_t off_rows, off_qf, off_lists, off_flags, total;
+    int64_t off_rows, off_qf, off_flags, off_pages, min_pages, total;
 };
+
+static int64_t split_page_floats(int64_t pages) {  // group counts (+ total), then 256 B aligned records
+    return (pages + 1 + 63) / 64 * 64 + pages * (RW * SP_PAGE);
+}
 
 typedef void (*PairsKernel)(RenderArgs, float*, int, float*);
 
@@ -3565,15 +3615,15 @@ static int split_plan(int ns, int cid, int64_t n_rays, int S, int PG, SplitPlan*
     sp->nb2 = (int64_t)g_num_cu * (per_cu < 1 ? 1 : per_cu);
     if (bwd_blocks(sp->kf, sp->bsf, n_rays, &sp->nbf)) return -1;
     const int64_t tot = (int64_t)S * PG;
-    // a MODE 2 wavefront takes rays wid, wid + nw, ...: at most rpw of them
-    const int64_t nw = sp->nb1 * SPLIT_WAVES, rpw = (n_rays + nw - 1) / nw;
-    sp->cap = (rpw * g_tune[TUNE_SPLIT_CAP] + 63) / 64 * 64;
+    // the records asked for, and one partly filled page per wavefront and family
+    sp->min_pages = (NCLASS * n_rays * g_tune[TUNE_SPLIT_CAP] + SP_PAGE - 1) / SP_PAGE +
+                    NCLASS * sp->nb1 * SPLIT_WAVES;
     sp->off_rows = 0;
     sp->off_qf = (sp->nb2 + 1) * tot;
-    sp->off_lists = sp->off_qf + sp->nbf * sp->bsf.waves * ring_floats_per_wave();
-    sp->off_flags = sp->off_lists + (int64_t)NCLASS * nw * RW * sp->cap;
-    sp->total = sp->off_flags + ((int64_t)NCLASS * nw + 1) + 1 + n_rays;  // counts + total, overflow, ray flags
-    sp->ok = true;
+    sp->off_flags = sp->off_qf + sp->nbf * sp->bsf.waves * ring_floats_per_wave();
+    sp->off_pages = (sp->off_flags + 1 + n_rays + 63) / 64 * 64;
+    sp->total = sp->off_pages + split_page_floats(sp->min_pages);
+    sp->ok = sp->min_pages < (1 << 30);
     return N3DS_OK;
 }
 
@@ -3665,23 +3715,25 @@ static int render_backward_impl(const float* origins, const float* directions, c
         if (st) return st;
         if (sp.ok && workspace_floats >= sp.total) {
             float* rows = workspace + sp.off_rows;
-            const int64_t nw = sp.nb1 * SPLIT_WAVES;
-            A.sp_list = workspace + sp.off_lists;
-            A.sp_count = (int*)(workspace + sp.off_flags);
-            A.sp_ovf = A.sp_count + NCLASS * nw + 1;
-            A.fbflag = A.sp_ovf + 1;
-            A.sp_cap = sp.cap;
-            A.sp_nw = (int)nw;
-            // the overflow flag and the ray flags start clear (every MODE 2 wavefront writes
-            // its own counts)
+            // every page the workspace holds: a caller that expects more live pairs gives more
+            int64_t pages = (workspace_floats - sp.off_pages - 64) / (RW * SP_PAGE + 1);
+            pages = std::min<int64_t>(std::max(pages, sp.min_pages), (1 << 30));
+            A.sp_next = (int*)(workspace + sp.off_flags);
+            A.fbflag = A.sp_next + 1;
+            A.sp_count = (int*)(workspace + sp.off_pages);
+            A.sp_list = workspace + sp.off_pages + (pages + 1 + 63) / 64 * 64;
+            A.sp_pages = (int)pages;
+            A.sp_first = (int)(NCLASS * sp.nb1 * SPLIT_WAVES);
+            // the page counter and the ray flags start clear (a wavefront writes the counts of
+            // the pages it took)
             const int64_t nflag = 1 + n_rays;
             hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)((nflag + 255) / 256)), dim3(256), 0, s,
-                               (float*)A.sp_ovf, nflag);
+                               (float*)A.sp_next, nflag);
             N3DS_LAUNCH_CHECK();
             hipLaunchKernelGGL(sp.k1, dim3((unsigned)sp.nb1), dim3(64 * SPLIT_WAVES), (size_t)sp.lds1, s, A, grad_rgb,
                                grad_acc, grad_depth, state, (float*)nullptr, 0, (float*)nullptr, (float*)nullptr);
             N3DS_LAUNCH_CHECK();
-            hipLaunchKernelGGL(group_scan_kernel, dim3(1), dim3(1024), 0, s, A.sp_count, (int64_t)NCLASS * nw,
+            hipLaunchKernelGGL(page_scan_kernel, dim3(1), dim3(SCAN_THREADS), 0, s, A.sp_count, A.sp_next, A.sp_first, A.sp_pages,
                                rows + sp.nb2 * tot, tot);
             N3DS_LAUNCH_CHECK();
             hipLaunchKernelGGL(pairs_kernel_ptr(color_id), dim3((unsigned)sp.nb2), dim3(64 * sp.pw), (size_t)sp.lds2,

@@ -63,26 +63,38 @@ def _check_device_ids(stroke_ids, Pmax, status):
 # alpha of each evaluated (sample, stroke) pair so the backward neither culls nor
 # evaluates alpha again; a ray that outgrows its capacity falls back to
 # recomputation chunk by chunk.  Capacities per ray: hits min(S, 2n), pairs 8n.
+# The Laplace transfer's tail reaches several stroke widths (7 to 12 n live pairs
+# per ray were counted on fields of 150 to 300 solids, 0.2 to 0.4 n with the linear
+# transfer), so it keeps 8n hits and 32n pairs where those fit the budget.
 STORE_BUDGET_BYTES = 8 << 30
 
 
-def keep_capacities(R, n, S, color_id):
-    cap_h = max(1, min(S, 2 * n))
-    cap_p = 8 * n
+def keep_capacities(R, n, S, color_id, wide=False):
+    cap_h = max(1, min(S, (8 if wide else 2) * n))
+    cap_p = (32 if wide else 8) * n
     npf = 4 if color_id == 1 else 1
     nch = (S + 63) // 64
     nbytes = R * (cap_h * 16 + cap_p * npf * 4 + nch * 12)
     return cap_h, cap_p, npf, nch, nbytes
 
 
-def _keep_buffers(store, R, n, S, color_id, dev):
+def _split_records(R, n, laplace):
+    """Floats of adjoint records beyond the library's default to make room for in the
+    backward's workspace: 16n live pairs of 8 floats per ray with the Laplace transfer,
+    up to half of the kept activations' budget."""
+    return min(R * n * 16 * 8, STORE_BUDGET_BYTES // 8) if laplace else 0
+
+
+def _keep_buffers(store, R, n, S, color_id, laplace, dev):
     if store is False:
         return None
     if isinstance(store, tuple):
         cap_h, cap_p = store
         npf, nch = (4 if color_id == 1 else 1), (S + 63) // 64
     else:
-        cap_h, cap_p, npf, nch, nbytes = keep_capacities(R, n, S, color_id)
+        cap_h, cap_p, npf, nch, nbytes = keep_capacities(R, n, S, color_id, laplace)
+        if laplace and nbytes > STORE_BUDGET_BYTES:
+            cap_h, cap_p, npf, nch, nbytes = keep_capacities(R, n, S, color_id)
         if store == 'auto' and nbytes > STORE_BUDGET_BYTES:
             return None
     return (torch.empty(R * nch * 3, dtype=torch.int32, device=dev),
@@ -122,7 +134,7 @@ def _launch_forward(origins, directions, viewdirs, radii, tdist, stroke_ids, sha
     depth = torch.empty(R, dtype=torch.float32, device=dev)
     state = torch.empty(5, R * (n1 - 1), dtype=torch.float32, device=dev)
     s_keep = S if scenes is None else scenes.s_max  # kept-hit layout follows the largest scene
-    keep = _keep_buffers(store, R, n1 - 1, s_keep, color_id, dev) if need_grad else None
+    keep = _keep_buffers(store, R, n1 - 1, s_keep, color_id, laplace, dev) if need_grad else None
     hd, hb, pb, cap_h, cap_p = keep if keep is not None else (None, None, None, 0, 0)
     if scenes is None:
         fwd, batch_args = _lib.lib().n3ds_render_forward, ()
@@ -184,7 +196,7 @@ class _render_fn(Function):
             nws = _lib.lib().n3ds_render_backward_workspace_floats(R, S, Pmax, Q)
             if hd.numel() > 0 and nws >= 0:  # kept hits: room for the split adjoint
                 nsp = _lib.lib().n3ds_render_backward_split_floats(R, S, Pmax, Q)
-                nws = -1 if nsp < 0 else max(nws, nsp)
+                nws = -1 if nsp < 0 else max(nws, nsp + (_split_records(R, n1 - 1, laplace) if nsp else 0))
             bwd, batch_args = _lib.lib().n3ds_render_backward, ()
         else:
             nws = _lib.lib().n3ds_render_batch_backward_workspace_floats(scenes.host_ptr(), scenes.n_scenes, n1 - 1,
