@@ -633,6 +633,503 @@ __global__ __launch_bounds__(GB_THREADS) void grid_bucket_reduce_kernel(GridBuck
     }
 }
 
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// ---------------------------------------------------------------------------
+// Table-gradient scatter by sorted tiles (hash grids in 3 dimensions).  The bucketed
+// scatter above lists 8 records of 4 + 4 C bytes per (point, level), placed one by one,
+// and adds them with LDS float atomics, which this card runs at one lane per three
+// clocks per CU (measured; 64-bit float atomics: 2.1 lanes per clock, whatever the
+// addresses).  Here
+//   1. sort: a block per (tile of 1024 points, level) sorts the tile's hits by bucket in
+//      LDS and writes them in that order, coalesced: a hit is one of the 4 (y, z) corner
+//      pairs of a point, whose two x corners always share a bucket (the hash multiplies
+//      x by 1, so x moves only the row's low bits; a dense level's buckets are whole
+//      lines of x), 8 + 4 C bytes: both rows within the bucket, the fraction in x and
+//      the upstream gradient times the pair's weight;
+//   2. add:  a block per bucket, whose rows it keeps in LDS as doubles (128 KB, one
+//      block per CU), streams its segment of every tile and adds both corners;
+//   3. sum:  the parts' copies of a level added into the gradient table (a level taken
+//      in one part adds to the table itself).
+// Gathering each hit's point and gradient in the add pass instead of writing them out
+// was slower: one lane per clock and CU (2^20 points x 16 levels x 2 features: 0.67 ms
+// of gathers in place of 16 bytes per hit written and read).  A level that fits neither
+// form (a hashed level of a size that is no power of two, say) adds with float atomics
+// to the table.
+// ---------------------------------------------------------------------------
+constexpr int GS_THREADS = 1024;
+constexpr int GS_WAVES = GS_THREADS / 64;
+constexpr int GS_TILE = 1024;             // points per sorted tile
+constexpr int GS_HITS = 4 * GS_TILE;      // hits per tile at most
+constexpr int GS_SORT_THREADS = 512;
+constexpr int GS_MAX_NB = 512;            // buckets per level
+constexpr int GS_XCD = 8;
+
+__host__ __device__ constexpr int gs_rows(int C) { return 16384 / C; }  // rows of a bucket: 128 KB of doubles
+
+enum { GS_NONE = 0, GS_HASH = 1, GS_DENSE = 2, GS_DIRECT = 3 };
+
+struct GsLevel {
+    int row0, hs, mode, nb;  // first row, rows, form, buckets
+    int rows;                // rows that corners can reach (a dense level's table is padded)
+    int lines;               // GS_DENSE: lines of x per bucket
+    uint32_t R;              // lattice points per axis
+};
+
+__device__ __forceinline__ GsLevel gs_level(const int* __restrict__ offsets, float scale, int level, int RB) {
+    GsLevel v;
+    v.row0 = offsets[level];
+    v.hs = offsets[level + 1] - v.row0;
+    v.R = (uint32_t)ceilf(scale) + 2u;
+    v.rows = v.hs;
+    v.lines = 0;
+    v.nb = 1;
+    if (v.hs <= 0) {
+        v.mode = GS_NONE;
+        v.nb = 0;
+        return v;
+    }
+    v.mode = GS_DIRECT;
+    if (v.R > (uint32_t)RB) return v;
+    const uint64_t R2 = (uint64_t)v.R * v.R, hs = (uint64_t)v.hs;
+    uint32_t stride = 1;  // grid_index's strides, wrapping like it
+    for (int d = 0; d < 3; d++)
+        if (stride <= (uint32_t)v.hs) stride *= v.R;
+    if (R2 * v.R <= hs) {
+        v.lines = RB / (int)v.R;
+        const int nb = ((int)R2 + v.lines - 1) / v.lines;
+        if (nb <= GS_MAX_NB) {
+            v.mode = GS_DENSE;
+            v.nb = nb;
+            v.rows = (int)(R2 * v.R);
+        }
+    } else if (stride > (uint32_t)v.hs && (hs & (hs - 1)) == 0 && v.hs / RB <= GS_MAX_NB) {
+        v.mode = GS_HASH;
+        v.nb = v.hs > RB ? v.hs / RB : 1;
+    }
+    return v;
+}
+
+// Parts the points are taken in: one for a level of 64 buckets or more (a part more costs a
+// copy of the level's rows written and read: 72 us for 2 parts of 16 levels at 2^20 points),
+// else about 128 blocks per level, whose short items fill in behind the long ones, with at
+// least 16384 hits each.
+__host__ __device__ inline int gs_parts(int64_t B, int nb) {
+    if (nb >= 64) return 1;
+    int64_t p = (128 + nb - 1) / nb;
+    const int64_t most = B / ((int64_t)4096 * nb);
+    if (p > most) p = most;
+    return p < 1 ? 1 : (int)p;
+}
+
+struct GsWs {
+    uint32_t* hits;  // [L, 2 + C, tiles * GS_HITS]: rows (first | second << 16), x fraction, values
+    uint32_t* segs;  // [L, GS_MAX_NB, tiles] first hit << 16 | hits
+    int* next;       // items of the add pass handed out
+    float* copies;   // parts of the levels taken in several, level after level
+    int tiles;
+};
+
+static int64_t gs_tiles(int64_t B) { return (B + GS_TILE - 1) / GS_TILE; }
+
+// bound on the copies' rows: a level taken in parts has at most 63 buckets
+static int64_t gs_copy_rows(int64_t B, int C, int L) {
+    const int64_t most = B / 4096;
+    return most > 1 ? (int64_t)L * gs_rows(C) * (most < 191 ? most : 191) : 0;
+}
+
+static int64_t gs_workspace_bytes(int64_t B, int C, int L) {
+    return gs_tiles(B) * L * (GS_HITS * 4 * (2 + C) + GS_MAX_NB * 4) + 256 + gs_copy_rows(B, C, L) * C * 4;
+}
+
+static GsWs gs_carve(void* ws, int64_t B, int C, int L) {
+    GsWs w;
+    w.tiles = (int)gs_tiles(B);
+    w.hits = (uint32_t*)ws;
+    w.segs = w.hits + (int64_t)w.tiles * L * GS_HITS * (2 + C);
+    w.next = (int*)(w.segs + (int64_t)w.tiles * L * GS_MAX_NB);
+    w.copies = (float*)(w.next + 64);
+    return w;
+}
+
+// Lattices wider than a bucket do not fit (their x moves the row out of it), and past 256
+// buckets per level the tiles' segments get much shorter than a wavefront.
+static bool gs_applies(int64_t B, int D, int C, int L, int64_t n_rows, int gridtype, int align, const LevelTab& lt) {
+    if (D != 3 || gridtype != 0 || align || B >= (1ll << 28) || n_rows > (int64_t)256 * L * gs_rows(C)) return false;
+    for (int l = 0; l < L; l++)
+        if (!(lt.scale[l] + 3.f < (float)gs_rows(C))) return false;
+    return true;
+}
+
+// points are padded by one per 32 in LDS (a wavefront reads them 32 apart)
+constexpr int GS_PAD_TILE = GS_TILE + GS_TILE / 32;
+__host__ __device__ constexpr int gs_sort_lds(int C) { return GS_PAD_TILE * 4 * (3 + C) + GS_HITS * 4; }
+
+template <typename T, int C>
+__global__ __launch_bounds__(GS_SORT_THREADS) void gs_sort_kernel(const T* __restrict__ grad,
+                                                                  const float* __restrict__ inputs,
+                                                                  const int* __restrict__ offsets, int64_t B, int L,
+                                                                  LevelTab lt, int interp, GsWs ws,
+                                                                  float* __restrict__ ggrid) {
+    constexpr int RB = gs_rows(C), PT = GS_TILE / GS_SORT_THREADS;
+    extern __shared__ float sm[];
+    float* sx = sm;                           // [3, GS_PAD_TILE] points, then their cell fractions
+    float* sg = sm + 3 * GS_PAD_TILE;         // [C, GS_PAD_TILE]
+    uint32_t* sorted = (uint32_t*)(sg + C * GS_PAD_TILE);  // [GS_HITS] point | pair << 10 | row << 12 | span << 26
+    static_assert(GS_TILE == 1 << 10 && gs_rows(1) <= 1 << 14, "a sorted hit is one word");
+    __shared__ int count[GS_MAX_NB];
+    __shared__ int wsum[GS_MAX_NB / 64];
+    static_assert(GS_MAX_NB == GS_SORT_THREADS, "one bucket per thread in the scan");
+    const int t = threadIdx.x, lane = t & 63;
+    if (blockIdx.x == 0 && t == 0) *ws.next = 0;
+    // a tile's levels run next to each other on one XCD (blocks go to XCDs round robin), so
+    // that its L2 serves the rows of the upstream gradient, which hold every level
+    const int64_t group = blockIdx.x / (GS_XCD * L);
+    const int rest = (int)(blockIdx.x - group * (GS_XCD * L));
+    const int64_t tile = group * GS_XCD + rest % GS_XCD;
+    const int level = rest / GS_XCD;
+    if (tile >= ws.tiles) return;
+    const GsLevel v = gs_level(offsets, lt.scale[level], level, RB);
+    if (v.mode == GS_NONE) return;
+    const int64_t b0 = tile * GS_TILE;
+    const int LC = L * C;
+    if (v.mode == GS_DIRECT) {
+        float* gg = ggrid + (int64_t)v.row0 * C;
+        for (int64_t b = b0 + t; b < min(B, b0 + GS_TILE); b += GS_SORT_THREADS) {
+            float pos[3], deriv[3];
+            uint32_t pg[3];
+            const LevelCoord lc = level_coords<3>(inputs + b * 3, level, offsets, lt, false, interp, pos, deriv, pg);
+            if (lc.oob) continue;
+            for (int corner = 0; corner < 8; corner++) {
+                float w = 1.f;
+                uint32_t loc[3];
+#pragma unroll
+                for (int d = 0; d < 3; d++) {
+                    if (corner & (1 << d)) { w *= pos[d]; loc[d] = pg[d] + 1; }
+                    else { w *= 1.f - pos[d]; loc[d] = pg[d]; }
+                }
+                const int64_t r = grid_index<3>(0, false, lc.hs, lc.res, loc);
+#pragma unroll
+                for (int c = 0; c < C; c++) atomicAdd(&gg[r * C + c], w * to_f<T>(grad[b * LC + level * C + c]));
+            }
+        }
+        return;
+    }
+    const float inv_lines = v.mode == GS_DENSE ? 1.f / (float)v.lines : 0.f;
+    // bucket of a line of x and the line's place in it (lines < 2^24: exact after one step)
+    auto line_bucket = [&](uint32_t ln, uint32_t& in_bucket) {
+        uint32_t q = (uint32_t)((float)ln * inv_lines);
+        if (q * (uint32_t)v.lines > ln) q--;
+        else if ((q + 1u) * (uint32_t)v.lines <= ln) q++;
+        in_bucket = ln - q * (uint32_t)v.lines;
+        return q;
+    };
+    const uint32_t mask = (uint32_t)min(v.hs, RB) - 1u;  // GS_HASH: row within the bucket
+    count[t] = 0;
+    const int np = (int)min((int64_t)GS_TILE, B - b0);
+    for (int i = t; i < 3 * np; i += GS_SORT_THREADS) {
+        const int p = i / 3;
+        sx[(i - 3 * p) * GS_PAD_TILE + p + (p >> 5)] = inputs[b0 * 3 + i];
+    }
+    for (int p = t; p < np; p += GS_SORT_THREADS)
+#pragma unroll
+        for (int c = 0; c < C; c++)
+            sg[c * GS_PAD_TILE + p + (p >> 5)] = to_f<T>(grad[(b0 + p) * LC + level * C + c]);
+    __syncthreads();
+    // the lanes of a wavefront take points 32 apart, so that neighbours in a bucket's order
+    // lie in different cells when the points are samples along rays (equal LDS addresses
+    // are added one by one)
+    uint32_t at[PT][4], row[PT][4];  // bucket << 16 | rank within the bucket; row within it | span << 14
+#pragma unroll
+    for (int i = 0; i < PT; i++) {
+        const int p = lane * (GS_TILE / 64) + (t >> 6) * PT + i, pp = p + (p >> 5);
+        bool on = p < np;
+        float in[3] = {-1.f, -1.f, -1.f}, pos[3], deriv[3];
+        uint32_t pg[3];
+        if (on) {
+#pragma unroll
+            for (int d = 0; d < 3; d++) in[d] = sx[d * GS_PAD_TILE + pp];
+        }
+        const LevelCoord lc = level_coords<3>(in, level, offsets, lt, false, interp, pos, deriv, pg);
+        on = on && !lc.oob;
+        if (on) {
+#pragma unroll
+            for (int d = 0; d < 3; d++) sx[d * GS_PAD_TILE + pp] = pos[d];
+        }
+        // the rows of x and x + 1 differ by the bits up to x's lowest zero bit
+        const uint32_t span = (uint32_t)min(__builtin_ctz(~pg[0]), 13);
+        const uint32_t hy = pg[1] * 2654435761u, hz = pg[2] * 805459861u;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            at[i][c] = ~0u;
+            row[i][c] = 0;
+            if (on) {
+                uint32_t id;
+                if (v.mode == GS_HASH) {
+                    const uint32_t h = pg[0] ^ ((c & 1) ? hy + 2654435761u : hy) ^ ((c >> 1) ? hz + 805459861u : hz);
+                    id = (h & ((uint32_t)v.hs - 1u)) / (uint32_t)RB;
+                    row[i][c] = (h & mask) | (span << 14);
+                } else {
+                    uint32_t in_bucket;
+                    id = line_bucket(pg[1] + (c & 1) + (pg[2] + (c >> 1)) * v.R, in_bucket);
+                    row[i][c] = pg[0] + in_bucket * v.R;
+                }
+                at[i][c] = (id << 16) | (uint32_t)atomicAdd(&count[id], 1);
+            }
+        }
+    }
+    __syncthreads();
+    // exclusive prefix of the bucket counts
+    const int own = count[t];
+    int incl = own;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int u = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += u;
+    }
+    if (lane == 63) wsum[t >> 6] = incl;
+    __syncthreads();
+    int start = incl - own, total = 0;
+#pragma unroll
+    for (int q = 0; q < GS_MAX_NB / 64; q++) {
+        if (q < (t >> 6)) start += wsum[q];
+        total += wsum[q];
+    }
+    count[t] = start;
+    if (t < v.nb)
+        ws.segs[((int64_t)level * GS_MAX_NB + t) * ws.tiles + tile] = ((uint32_t)start << 16) | (uint32_t)own;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < PT; i++)
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+            if (at[i][c] != ~0u)
+                sorted[count[at[i][c] >> 16] + (at[i][c] & 0xffffu)] =
+                    (uint32_t)(lane * (GS_TILE / 64) + (t >> 6) * PT + i) | (c << 10) | (row[i][c] << 12);
+    __syncthreads();
+    const int64_t plane = (int64_t)ws.tiles * GS_HITS;
+    uint32_t* dst = ws.hits + (int64_t)level * (2 + C) * plane + tile * GS_HITS;
+    for (int i = t; i < total; i += GS_SORT_THREADS) {
+        const uint32_t e = sorted[i], p = e & (GS_TILE - 1), pp = p + (p >> 5);
+        const uint32_t r0 = (e >> 12) & 0x3fffu;
+        const uint32_t r1 = v.mode == GS_HASH ? r0 ^ (((2u << (e >> 26)) - 1u) & mask) : r0 + 1u;
+        const float wy = sx[GS_PAD_TILE + pp], wz = sx[2 * GS_PAD_TILE + pp];
+        const float w = ((e & (1u << 10)) ? wy : 1.f - wy) * ((e & (1u << 11)) ? wz : 1.f - wz);
+        dst[i] = r0 | (r1 << 16);
+        dst[plane + i] = __float_as_uint(sx[pp]);
+#pragma unroll
+        for (int c = 0; c < C; c++) dst[(2 + c) * plane + i] = __float_as_uint(w * sg[c * GS_PAD_TILE + pp]);
+    }
+}
+
+// One bucket of one level over one part of the tiles; copy: the first row of the level's
+// copies (-1: the only part, which adds to the table itself).
+template <int C>
+__device__ __forceinline__ void gs_add_item(const int* __restrict__ offsets, int64_t B, const LevelTab& lt,
+                                            const GsWs& ws, float* __restrict__ ggrid, int level, int part, int bucket,
+                                            int64_t copy, double* acc, int t, int lane, int wave) {
+    constexpr int RB = gs_rows(C), U = 4;
+    const GsLevel v = gs_level(offsets, lt.scale[level], level, RB);
+    const int parts = gs_parts(B, v.nb);
+    const int per = (ws.tiles + parts - 1) / parts;
+    const int t0 = min(ws.tiles, per * part), t1 = min(ws.tiles, t0 + per);
+    const int first_row = v.mode == GS_DENSE ? bucket * v.lines * (int)v.R : bucket * RB;
+    const int nrow = min(v.rows - first_row, v.mode == GS_DENSE ? v.lines * (int)v.R : RB);
+    for (int i = t; i < RB * C; i += GS_THREADS) acc[i] = 0.0;
+    __syncthreads();
+    // a wavefront takes every GS_WAVES-th tile, 64 of them at a time: lane l holds the l-th
+    // one's segment, and the segments are walked end to end in full wavefronts
+    const uint32_t* segs = ws.segs + ((int64_t)level * GS_MAX_NB + bucket) * ws.tiles;
+    const int64_t plane = (int64_t)ws.tiles * GS_HITS;
+    const uint32_t* hits = ws.hits + (int64_t)level * (2 + C) * plane;
+    for (int base = t0 + wave; base < t1; base += 64 * GS_WAVES) {
+        const int tile = base + lane * GS_WAVES;
+        const uint32_t sg = tile < t1 ? segs[tile] : 0u;
+        const int n = (int)(sg & 0xffffu);
+        int end = n;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int u = __shfl_up(end, off, 64);
+            if (lane >= off) end += u;
+        }
+        const int total = __builtin_amdgcn_readlane(end, 63);
+        const int shift = tile * GS_HITS + (int)(sg >> 16) - (end - n);  // hit of position p: shift + p
+        int j = 0, ej = __builtin_amdgcn_readlane(end, 0), oj = __builtin_amdgcn_readlane(shift, 0);
+        for (int i0 = 0; i0 < total; i0 += 64 * U) {
+            int at[U];
+#pragma unroll
+            for (int q = 0; q < U; q++) {
+                const int p = i0 + 64 * q + lane;
+                at[q] = oj;
+                while (j < 63 && ej <= i0 + 64 * q + 63) {  // the segment ends within this wavefront's 64
+                    j++;
+                    oj = __builtin_amdgcn_readlane(shift, j);
+                    if (p >= ej) at[q] = oj;
+                    ej = __builtin_amdgcn_readlane(end, j);
+                }
+                at[q] = p < total ? at[q] + p : -1;
+            }
+            uint32_t rr[U];
+            float fx[U], val[U][C];
+#pragma unroll
+            for (int q = 0; q < U; q++)
+                if (at[q] >= 0) {
+                    const uint32_t* h = hits + at[q];
+                    rr[q] = h[0];
+                    fx[q] = __uint_as_float(h[plane]);
+#pragma unroll
+                    for (int c = 0; c < C; c++) val[q][c] = __uint_as_float(h[(2 + c) * plane]);
+                }
+#pragma unroll
+            for (int q = 0; q < U; q++)
+                if (at[q] >= 0) {
+#pragma unroll
+                    for (int c = 0; c < C; c++) {
+                        atomicAdd(&acc[c * RB + (rr[q] & 0xffffu)], (double)((1.f - fx[q]) * val[q][c]));
+                        atomicAdd(&acc[c * RB + (rr[q] >> 16)], (double)(fx[q] * val[q][c]));
+                    }
+                }
+        }
+    }
+    __syncthreads();
+    if (copy < 0) {  // the only part: the bucket's rows belong to this block
+        float* dst = ggrid + ((int64_t)v.row0 + first_row) * C;
+        for (int i = t; i < nrow * C; i += GS_THREADS) {
+            const float a = (float)acc[(i % C) * RB + i / C];
+            if (a != 0.f) dst[i] += a;
+        }
+    } else {
+        float* dst = ws.copies + (copy + (int64_t)part * v.rows + first_row) * C;
+        for (int i = t; i < nrow * C; i += GS_THREADS) dst[i] = (float)acc[(i % C) * RB + i / C];
+    }
+}
+
+template <int C>
+__global__ __launch_bounds__(GS_THREADS) void gs_add_kernel(const int* __restrict__ offsets, int64_t B, int L,
+                                                            LevelTab lt, GsWs ws, float* __restrict__ ggrid) {
+    extern __shared__ double acc[];  // [C, RB]
+    __shared__ int pick[3];
+    __shared__ int64_t pick_copy;
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    // items (level, part, bucket), the finest level first: its few long items start early and
+    // the coarse levels' many short ones fill in behind; lane l holds the l-th one's place
+    const int mine = L - 1 - lane;
+    GsLevel v;
+    v.nb = 0;
+    v.rows = 0;
+    v.mode = GS_NONE;
+    int parts = 0;
+    if (lane < L) {
+        v = gs_level(offsets, lt.scale[mine], mine, gs_rows(C));
+        if (v.nb > 0 && v.mode != GS_DIRECT) parts = gs_parts(B, v.nb);
+    }
+    int64_t cincl = parts > 1 ? (int64_t)parts * v.rows : 0;
+    const int64_t cown = cincl;
+    int iincl = parts * v.nb;
+    const int iown = iincl;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int u = __shfl_up(iincl, off, 64);
+        const int64_t cu = __shfl_up(cincl, off, 64);
+        if (lane >= off) {
+            iincl += u;
+            cincl += cu;
+        }
+    }
+    for (bool first = true;; first = false) {
+        if (wave == 0) {
+            // the next item, taken as the blocks get done
+            int s = blockIdx.x;
+            if (!first) {
+                if (lane == 0) s = (int)gridDim.x + atomicAdd(ws.next, 1);
+                s = __builtin_amdgcn_readfirstlane(s);
+            }
+            const int at = s - (iincl - iown);
+            if (lane == 0) pick[0] = -1;
+            wave_fence();
+            if (at >= 0 && at < iown) {
+                pick[0] = mine;
+                pick[1] = at / v.nb;
+                pick[2] = at % v.nb;
+                pick_copy = parts > 1 ? cincl - cown : -1;
+            }
+        }
+        __syncthreads();
+        const int level = __builtin_amdgcn_readfirstlane(pick[0]);
+        if (level < 0) return;  // past the last item
+        const int part = __builtin_amdgcn_readfirstlane(pick[1]), bucket = __builtin_amdgcn_readfirstlane(pick[2]);
+        gs_add_item<C>(offsets, B, lt, ws, ggrid, level, part, bucket, pick_copy, acc, t, lane, wave);
+        __syncthreads();
+    }
+}
+
+// ggrid += the parts' copies.  blockIdx.y = level.
+template <int C>
+__global__ __launch_bounds__(256) void gs_sum_kernel(const int* __restrict__ offsets, int64_t B, int L, LevelTab lt,
+                                                     GsWs ws, float* __restrict__ ggrid) {
+    constexpr int RB = gs_rows(C);
+    const int level = blockIdx.y;
+    const GsLevel v = gs_level(offsets, lt.scale[level], level, RB);
+    if (v.nb == 0 || v.mode == GS_DIRECT) return;
+    const int parts = gs_parts(B, v.nb);
+    if (parts == 1) return;
+    int64_t copy = 0;  // rows of the finer levels, whose copies come first
+    for (int l = L - 1; l > level; l--) {
+        const GsLevel u = gs_level(offsets, lt.scale[l], l, RB);
+        const int p = u.nb > 0 && u.mode != GS_DIRECT ? gs_parts(B, u.nb) : 0;
+        if (p > 1) copy += (int64_t)p * u.rows;
+    }
+    const int64_t n = (int64_t)v.rows * C;
+    const float* src = ws.copies + copy * C;
+    float* dst = ggrid + (int64_t)v.row0 * C;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        float a = 0.f;
+#pragma unroll 8
+        for (int p = 0; p < parts; p++) a += src[p * n + i];
+        if (a != 0.f) dst[i] += a;
+    }
+}
+
+static int g_pf_cu = 0;
+
+static int prop_blocks(int64_t work, int threads, int per_cu, int64_t* out) {
+    if (g_pf_cu == 0) {
+        int dev;
+        N3DS_HIP_CHECK(hipGetDevice(&dev));
+        N3DS_HIP_CHECK(hipDeviceGetAttribute(&g_pf_cu, hipDeviceAttributeMultiprocessorCount, dev));
+    }
+    int64_t nb = (work + threads - 1) / threads;
+    const int64_t cap = (int64_t)g_pf_cu * per_cu;
+    *out = nb < 1 ? 1 : (nb > cap ? cap : nb);
+    return N3DS_OK;
+}
+
+template <typename T, int C>
+static int gs_launch(const T* grad, const float* inputs, const int* offsets, int64_t B, int L, const LevelTab& lt,
+                     int interp, void* workspace, float* ggrid, hipStream_t s) {
+    const GsWs ws = gs_carve(workspace, B, C, L);
+    const size_t lds = (size_t)gs_rows(C) * C * 8;
+    N3DS_HIP_CHECK(hipFuncSetAttribute((const void*)gs_add_kernel<C>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       (int)lds));
+    N3DS_HIP_CHECK(hipFuncSetAttribute((const void*)gs_sort_kernel<T, C>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       gs_sort_lds(C)));
+    int64_t nb;
+    const int st = prop_blocks((int64_t)1 << 40, 1, 1, &nb);  // one persistent block per CU
+    if (st) return st;
+    const int64_t groups = (ws.tiles + GS_XCD - 1) / GS_XCD;
+    hipLaunchKernelGGL((gs_sort_kernel<T, C>), dim3((unsigned)(groups * GS_XCD * L)), dim3(GS_SORT_THREADS),
+                       gs_sort_lds(C), s, grad, inputs, offsets, B, L, lt, interp, ws, ggrid);
+    hipLaunchKernelGGL((gs_add_kernel<C>), dim3((unsigned)nb), dim3(GS_THREADS), lds, s, offsets, B, L, lt, ws, ggrid);
+    hipLaunchKernelGGL((gs_sum_kernel<C>), dim3(128, (unsigned)L), dim3(256), 0, s, offsets, B, L, lt, ws, ggrid);
+    N3DS_LAUNCH_CHECK();
+    return N3DS_OK;
+}
+
 // ---------------------------------------------------------------------------
 // Fused proposal density field: the reference's PropMLP forward
 // (source/models.py:286-523 with disable_rgb: _warp_coords, GridEncoder with
@@ -664,12 +1161,6 @@ struct PropArgs {
     const float* b2;  // [1]
     float dbias;
 };
-
-__device__ __forceinline__ void wave_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // models.py:19-33 and coord.contract (utils/coord.py:5-11), then grid.py:158
 // (inputs + bound) / (2 bound) with bound 1
@@ -941,7 +1432,10 @@ N3DS_EXPORT int n3ds_grid_encode_forward(const float* inputs, const void* embedd
 
 N3DS_EXPORT int64_t n3ds_grid_encode_backward_workspace_bytes(int64_t B, int D, int C, int L, int64_t n_rows) {
     if (B < 0 || D < 1 || D > 5 || C < 1 || C > 8 || L < 1 || n_rows < 0) return -1;
-    return gb_workspace_bytes(B, D, C, L, n_rows);
+    // either scatter (the grid type, alignment and scales are not known here)
+    const int64_t gb = gb_workspace_bytes(B, D, C, L, n_rows);
+    const int64_t gs = D == 3 ? gs_workspace_bytes(B, C, L) : 0;
+    return gb > gs ? gb : gs;
 }
 
 // grad_embeddings_f32: fp32 accumulation table (zero-initialised by the caller);
@@ -961,7 +1455,23 @@ N3DS_EXPORT int n3ds_grid_encode_backward(const void* grad, const float* inputs,
     const bool bucketed = workspace != nullptr;
     if (bucketed)
         N3DS_REQUIRE(workspace_bytes >= gb_workspace_bytes(B, D, C, L, n_rows), "grid workspace too small");
-    if (B > 0 && bucketed && n_rows > 0) {
+    const bool sorted = bucketed && gs_applies(B, D, C, L, n_rows, gridtype, align_corners, lt) &&
+                        workspace_bytes >= gs_workspace_bytes(B, C, L);
+    if (B > 0 && sorted && n_rows > 0) {
+#define LAUNCH_S(CC)                                                                                             \
+    st = dtype == 0 ? gs_launch<float, CC>((const float*)grad, inputs, offsets, B, L, lt, interp, workspace,     \
+                                           grad_embeddings_f32, s)                                               \
+                    : gs_launch<__half, CC>((const __half*)grad, inputs, offsets, B, L, lt, interp, workspace,   \
+                                            grad_embeddings_f32, s)
+        switch (C) {
+            case 1: LAUNCH_S(1); break;
+            case 2: LAUNCH_S(2); break;
+            case 4: LAUNCH_S(4); break;
+            default: LAUNCH_S(8); break;
+        }
+#undef LAUNCH_S
+        if (st) return st;
+    } else if (B > 0 && bucketed && n_rows > 0) {
         const GridBucketWs ws = gb_carve(workspace, B, D, C, L, n_rows);
         const int64_t NB = gb_num_buckets(n_rows, C);
         hipLaunchKernelGGL(grid_fill_int_kernel, dim3((unsigned)((NB + 255) / 256)), dim3(256), 0, s, ws.count, NB);
@@ -1060,20 +1570,6 @@ static int prop_check(int64_t N, int C, int L, int dtype, int warp) {
     N3DS_REQUIRE(L >= 1 && L * C <= PF_MAXF, "num_levels * level_dim must be in [1, %d] (got %d x %d)", PF_MAXF, L, C);
     N3DS_REQUIRE(dtype == 0 || dtype == 1, "dtype must be 0 (float32) or 1 (float16)");
     N3DS_REQUIRE(warp >= 0 && warp <= 2, "warp must be 0 (none), 1 (contract) or 2 (box)");
-    return N3DS_OK;
-}
-
-static int g_pf_cu = 0;
-
-static int prop_blocks(int64_t work, int threads, int per_cu, int64_t* out) {
-    if (g_pf_cu == 0) {
-        int dev;
-        N3DS_HIP_CHECK(hipGetDevice(&dev));
-        N3DS_HIP_CHECK(hipDeviceGetAttribute(&g_pf_cu, hipDeviceAttributeMultiprocessorCount, dev));
-    }
-    int64_t nb = (work + threads - 1) / threads;
-    const int64_t cap = (int64_t)g_pf_cu * per_cu;
-    *out = nb < 1 ? 1 : (nb > cap ? cap : nb);
     return N3DS_OK;
 }
 
