@@ -283,8 +283,8 @@ class _compositing_fn(Function):
         dev = alphas.device
         gd = torch.zeros(0, device=dev) if grad_density is None else _as_f32(grad_density, (-1,))
         gc = torch.zeros(0, device=dev) if grad_color is None else _as_f32(grad_color, (-1, colors.shape[-1]))
-        g_alpha = torch.zeros_like(alphas)
-        g_colors = torch.zeros_like(colors)
+        g_alpha = torch.empty_like(alphas)  # every element is written
+        g_colors = torch.empty_like(colors)
         g_dp = torch.zeros_like(density_params)
         _backend.compose_backward(g_alpha, g_colors, g_dp, gd, gc, alphas, colors, density_params, adjoint)
         return g_alpha.reshape(*pre_shape, n_str), g_colors.reshape(*pre_shape, n_str, colors.shape[-1]), g_dp
