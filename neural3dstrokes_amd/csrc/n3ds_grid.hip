@@ -53,6 +53,13 @@ __device__ __forceinline__ float from_f<float>(float v) { return v; }
 template <>
 __device__ __forceinline__ __half from_f<__half>(float v) { return __float2half(v); }
 
+// keeps a float32 result from being folded with its conversion to half into one rounding
+// (v_fma_mixlo_f16): results stay those of a float32 interpolation rounded once on store
+__device__ __forceinline__ float rounded(float v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
 struct LevelCoord {
     uint32_t hs, res;
     float scale;
@@ -132,7 +139,10 @@ __global__ __launch_bounds__(256) void grid_fwd_kernel(const float* __restrict__
         return;
     }
     const T* g = grid + (int64_t)offsets[level] * C;
-    float acc[C];
+    // every corner is gathered once: the slopes are differences of the same values (gathering
+    // them again for each axis, 24 more for D = 3, took 630 of the 943 us of a forward and
+    // adjoint with input gradients at 200003 points x 16 levels)
+    float acc[C], val[1 << D][C];
 #pragma unroll
     for (int c = 0; c < C; c++) acc[c] = 0.f;
 #pragma unroll
@@ -146,10 +156,13 @@ __global__ __launch_bounds__(256) void grid_fwd_kernel(const float* __restrict__
         }
         uint32_t idx = grid_index<D>(gridtype, align != 0, lc.hs, lc.res, loc) * C;
 #pragma unroll
-        for (int c = 0; c < C; c++) acc[c] += w * to_f<T>(g[idx + c]);
+        for (int c = 0; c < C; c++) {
+            val[corner][c] = to_f<T>(g[idx + c]);
+            acc[c] += w * val[corner][c];
+        }
     }
 #pragma unroll
-    for (int c = 0; c < C; c++) out[c] = from_f<T>(acc[c]);
+    for (int c = 0; c < C; c++) out[c] = from_f<T>(rounded(acc[c]));
     if (dy_dx) {
         T* dd = dy_dx + b * (int64_t)L * D * C + (int64_t)level * D * C;
 #pragma unroll
@@ -160,22 +173,18 @@ __global__ __launch_bounds__(256) void grid_fwd_kernel(const float* __restrict__
 #pragma unroll
             for (int corner = 0; corner < (1 << (D - 1)); corner++) {
                 float w = lc.scale;
-                uint32_t loc[D];
+                int left = 0;  // the corner with the axis's bit clear
 #pragma unroll
                 for (int nd = 0; nd < D - 1; nd++) {
-                    int d = nd >= gd ? nd + 1 : nd;
-                    if (corner & (1 << nd)) { w *= pos[d]; loc[d] = pg[d] + 1; }
-                    else { w *= 1.f - pos[d]; loc[d] = pg[d]; }
+                    const int d = nd >= gd ? nd + 1 : nd;
+                    if (corner & (1 << nd)) { w *= pos[d]; left |= 1 << d; }
+                    else { w *= 1.f - pos[d]; }
                 }
-                loc[gd] = pg[gd];
-                uint32_t il = grid_index<D>(gridtype, align != 0, lc.hs, lc.res, loc) * C;
-                loc[gd] = pg[gd] + 1;
-                uint32_t ir = grid_index<D>(gridtype, align != 0, lc.hs, lc.res, loc) * C;
 #pragma unroll
-                for (int c = 0; c < C; c++) rg[c] += w * (to_f<T>(g[ir + c]) - to_f<T>(g[il + c])) * deriv[gd];
+                for (int c = 0; c < C; c++) rg[c] += w * (val[left | (1 << gd)][c] - val[left][c]) * deriv[gd];
             }
 #pragma unroll
-            for (int c = 0; c < C; c++) dd[gd * C + c] = from_f<T>(rg[c]);
+            for (int c = 0; c < C; c++) dd[gd * C + c] = from_f<T>(rounded(rg[c]));
         }
     }
 }
@@ -1142,8 +1151,7 @@ static int gs_launch(const T* grad, const float* inputs, const int* offsets, int
 constexpr int PF_HID = 64;
 constexpr int PF_MAXF = 32;
 constexpr int PF_FWD_THREADS = 256;
-constexpr int PF_BWD_THREADS = 128;
-constexpr int PF_CH = 16;  // hidden units per weight-gradient chunk
+constexpr int PF_BWD_THREADS = 256;
 
 struct PropArgs {
     const float* coords;  // [N, 3] sample positions
@@ -1252,121 +1260,187 @@ __global__ __launch_bounds__(PF_FWD_THREADS) void prop_fwd_kernel(PropArgs P, fl
     }
 }
 
+typedef float f4 __attribute__((ext_vector_type(4)));
+
+// D = A B + C in float32 on the matrix cores: A 16 x 4 (lane l: row l % 16, column l / 16),
+// B 4 x 16 (lane l: column l % 16, row l / 16), C and D 16 x 16 (lane l: column l % 16, rows
+// 4 (l / 16) + 0..3).
+__device__ __forceinline__ f4 mfma16(float a, float b, f4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// Adjoint of the head.  Its three contractions (hidden units from features, feature
+// gradients from hidden gradients, weight gradients over the points) run on the matrix
+// cores in float32, 16 points at a time:
+//   H [hidden x point] = W1 F: the operands' lanes hold W1 and the features; a lane then has
+//     4 hidden units of one point per 16 x 16 tile, sums their W2 relu(H) for the density
+//     and turns them into dH in place, which is at once the right operand of
+//   dF [feature x point] = W1^T dH (the k-th step takes the hidden units 4 (l / 16) + k);
+//   H' [point x hidden] = the same product with its operands exchanged: dH' of it is the
+//     right operand of dW1 [feature x hidden] += F^T dH', summed over all of a wavefront's
+//     points in the accumulator registers.
+// 56 matrix instructions per 16 points and 10 features.  The vector version went through
+// LDS for every product (7 LDS reads per point and hidden unit): 1560 us at 4.2 M points.
 template <typename T, int C, int FM, int FX = 0>
 __global__ __launch_bounds__(PF_BWD_THREADS) void prop_bwd_kernel(PropArgs P, const float* __restrict__ gdens,
                                                                   const float* __restrict__ feat_in,
                                                                   float* __restrict__ gfeat, float* __restrict__ x01_out,
                                                                   float* __restrict__ gW1, float* __restrict__ gb1,
                                                                   float* __restrict__ gW2, float* __restrict__ gb2) {
-    constexpr int NW = PF_BWD_THREADS / 64;
-    __shared__ float sW1[PF_HID * PF_MAXF], sb1[PF_HID], sW2[PF_HID];
-    __shared__ float aW1[PF_HID * PF_MAXF], ab1[PF_HID], aW2[PF_HID], ab2[1];  // block accumulators
-    __shared__ float sf[NW][64][FM + 1];                                        // features, point-major
-    __shared__ float sdh[NW][64][PF_CH + 1], sh[NW][64][PF_CH + 1];            // one chunk of hidden units
-    __shared__ float sg[NW][64];
+    constexpr int NW = PF_BWD_THREADS / 64, KS = (FM + 3) / 4, FT = (FM + 15) / 16, HT = PF_HID / 16;
+    constexpr int FP = 16 * FT + 1;  // row of a point's features in LDS
+    __shared__ float sf[NW][64][FP];  // a wavefront's 64 points: features, then their gradients
+    __shared__ double sum[PF_HID * (FM + 2) + 1];  // dW1 [hidden, feature], db1, dW2, db2 of the block
     const int F = FX > 0 ? FX : P.L * C;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform per wavefront
-    for (int i = threadIdx.x; i < PF_HID * F; i += PF_BWD_THREADS) {
-        sW1[i] = P.W1[i];
-        aW1[i] = 0.f;
+    const int lc = lane & 15, lr = lane >> 4;
+    for (int i = threadIdx.x; i < PF_HID * (FM + 2) + 1; i += PF_BWD_THREADS) sum[i] = 0.0;
+    // constant operands: w1[t][k] = W1[16 t + lc][4 k + lr], w1t[q][t][r] = W1[16 t + 4 lr + r][16 q + lc]
+    float w1[HT][KS], w1t[FT][HT][4], b1q[HT], w2q[HT];
+    f4 b1p[HT], w2p[HT];
+#pragma unroll
+    for (int t = 0; t < HT; t++) {
+#pragma unroll
+        for (int k = 0; k < KS; k++) w1[t][k] = 4 * k + lr < F ? P.W1[(16 * t + lc) * F + 4 * k + lr] : 0.f;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int j = 16 * t + 4 * lr + r;
+#pragma unroll
+            for (int q = 0; q < FT; q++) w1t[q][t][r] = 16 * q + lc < F ? P.W1[j * F + 16 * q + lc] : 0.f;
+            b1p[t][r] = P.b1[j];
+            w2p[t][r] = P.W2[j];
+        }
+        b1q[t] = P.b1[16 * t + lc];
+        w2q[t] = P.W2[16 * t + lc];
     }
-    for (int i = threadIdx.x; i < PF_HID; i += PF_BWD_THREADS) {
-        sb1[i] = P.b1[i];
-        sW2[i] = P.W2[i];
-        ab1[i] = 0.f;
-        aW2[i] = 0.f;
-    }
-    if (threadIdx.x == 0) ab2[0] = 0.f;
-    __syncthreads();
     const float b2 = P.b2[0];
-    // every lane runs the same number of tiles (points past N contribute zeros)
-    const int64_t ntile = (P.N + PF_BWD_THREADS - 1) / PF_BWD_THREADS;
-    float gb2_lane = 0.f;
-    for (int64_t tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
-        const int64_t b = tile * PF_BWD_THREADS + threadIdx.x;
-        const bool live = b < P.N;
-        float f[FM], df[FM], g = 0.f;
+    f4 aw1[FT][HT];
+    float ab1[HT], aw2[HT], ab2 = 0.f;
 #pragma unroll
-        for (int i = 0; i < FM; i++) { f[i] = 0.f; df[i] = 0.f; }
-        if (live) {
-            if (feat_in) {
+    for (int t = 0; t < HT; t++) {
+        ab1[t] = aw2[t] = 0.f;
 #pragma unroll
-                for (int i = 0; i < FM; i++)
-                    if (i < F) f[i] = feat_in[b * F + i];
-            } else {
-                float cw[3], x01[3];
-                prop_warp(P, b, cw, x01);
+        for (int q = 0; q < FT; q++) aw1[q][t] = (f4){0.f, 0.f, 0.f, 0.f};
+    }
+    __syncthreads();
+    const int64_t ntile = (P.N + 63) / 64;
+    for (int64_t tile = (int64_t)blockIdx.x * NW + wave; tile < ntile; tile += (int64_t)gridDim.x * NW) {
+        const int64_t b0 = tile * 64;
+        const int np = (int)min((int64_t)64, P.N - b0);
+        float(*pt)[FP] = sf[wave];
+        if (feat_in) {
+            for (int i = lane; i < 64 * 16 * FT; i += 64) {
+                const int p = i / (16 * FT), c = i - p * (16 * FT);
+                if (c >= F || p >= np) pt[p][c] = 0.f;
+            }
+            for (int i = lane; i < np * F; i += 64) {
+                const int p = i / F;
+                pt[p][i - p * F] = feat_in[b0 * F + i];
+            }
+        } else {
+            float f[FM], cw[3], x01[3];
+#pragma unroll
+            for (int i = 0; i < FM; i++) f[i] = 0.f;
+            if (lane < np) {
+                prop_warp(P, b0 + lane, cw, x01);
                 prop_features<T, C, FM>(P, x01, f);
 #pragma unroll
-                for (int d = 0; d < 3; d++) x01_out[b * 3 + d] = x01[d];
+                for (int d = 0; d < 3; d++) x01_out[(b0 + lane) * 3 + d] = x01[d];
             }
-            const float raw = prop_raw<FM>(sW1, sb1, sW2, b2, F, f);
-            g = gdens[b] * dsoftplus20(raw + P.dbias);
+#pragma unroll
+            for (int i = 0; i < 16 * FT; i++) pt[lane][i] = i < FM && i < F ? f[i < FM ? i : 0] : 0.f;
         }
-        gb2_lane += g;
+        const float gown = lane < np ? gdens[b0 + lane] : 0.f;
+        wave_fence();
+#pragma unroll 1
+        for (int s = 0; s < 4; s++) {  // 16 points
+            float f[KS], ft[FT][4];
 #pragma unroll
-        for (int i = 0; i < FM; i++) sf[wave][lane][i] = f[i];
-        sg[wave][lane] = g;
-        for (int j0 = 0; j0 < PF_HID; j0 += PF_CH) {
-            // per point: the chunk's hidden units, their adjoints and dL/df
-#pragma unroll 4
-            for (int jj = 0; jj < PF_CH; jj++) {
-                const int j = j0 + jj;
-                float a = sb1[j];
+            for (int k = 0; k < KS; k++) f[k] = pt[16 * s + lc][4 * k + lr];
 #pragma unroll
-                for (int i = 0; i < FM; i++)
-                    if (i < F) a += sW1[j * F + i] * f[i];
-                const float dh = a > 0.f ? g * sW2[j] : 0.f;
+            for (int q = 0; q < FT; q++)
 #pragma unroll
-                for (int i = 0; i < FM; i++)
-                    if (i < F) df[i] += dh * sW1[j * F + i];
-                sdh[wave][lane][jj] = dh;
-                sh[wave][lane][jj] = fmaxf(a, 0.f);
+                for (int r = 0; r < 4; r++) ft[q][r] = pt[16 * s + 4 * lr + r][16 * q + lc];
+            f4 h[HT];
+#pragma unroll
+            for (int t = 0; t < HT; t++) {
+                h[t] = b1p[t];
+#pragma unroll
+                for (int k = 0; k < KS; k++) h[t] = mfma16(w1[t][k], f[k], h[t]);
             }
-            wave_fence();
-            // per hidden unit: sums over the wave's 64 points; lane = (unit jj, feature group ig)
-            constexpr int KG = FM / 4;  // features per lane group
-            const int jj = lane & (PF_CH - 1), ig = lane >> 4;  // 4 groups of KG features
-            float w1[KG], bsum = 0.f, w2 = 0.f;
+            float raw = 0.f;
 #pragma unroll
-            for (int k = 0; k < KG; k++) w1[k] = 0.f;
-            for (int q = 0; q < 64; q++) {
-                const float dh = sdh[wave][q][jj];
+            for (int t = 0; t < HT; t++)
 #pragma unroll
-                for (int k = 0; k < KG; k++) w1[k] += dh * sf[wave][q][ig * KG + k];
-                if (ig == 0) {
-                    bsum += dh;
-                    w2 += sg[wave][q] * sh[wave][q][jj];
+                for (int r = 0; r < 4; r++) raw += w2p[t][r] * fmaxf(h[t][r], 0.f);
+            raw += __shfl_xor(raw, 16, 64);
+            raw += __shfl_xor(raw, 32, 64);
+            const float g = __shfl(gown, 16 * s + lc, 64) * dsoftplus20(raw + b2 + P.dbias);
+            if (lr == 0) ab2 += g;
+            f4 df[FT];
+#pragma unroll
+            for (int q = 0; q < FT; q++) df[q] = (f4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int t = 0; t < HT; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const float dh = h[t][r] > 0.f ? g * w2p[t][r] : 0.f;
+#pragma unroll
+                    for (int q = 0; q < FT; q++) df[q] = mfma16(w1t[q][t][r], dh, df[q]);
+                }
+            float gq[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) gq[r] = __shfl(g, 4 * lr + r, 64);
+#pragma unroll
+            for (int t = 0; t < HT; t++) {
+                f4 hq = (f4){b1q[t], b1q[t], b1q[t], b1q[t]};
+#pragma unroll
+                for (int k = 0; k < KS; k++) hq = mfma16(f[k], w1[t][k], hq);
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const float dh = hq[r] > 0.f ? gq[r] * w2q[t] : 0.f;
+                    ab1[t] += dh;
+                    aw2[t] += gq[r] * fmaxf(hq[r], 0.f);
+#pragma unroll
+                    for (int q = 0; q < FT; q++) aw1[q][t] = mfma16(ft[q][r], dh, aw1[q][t]);
                 }
             }
-            const int j = j0 + jj;
+            // the points' features are done with: their gradients take the place
 #pragma unroll
-            for (int k = 0; k < KG; k++)
-                if (ig * KG + k < F) atomicAdd(&aW1[j * F + ig * KG + k], w1[k]);
-            if (ig == 0) {
-                atomicAdd(&ab1[j], bsum);
-                atomicAdd(&aW2[j], w2);
+            for (int q = 0; q < FT; q++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) pt[16 * s + lc][16 * q + 4 * lr + r] = df[q][r];
+        }
+        wave_fence();
+        for (int i = lane; i < np * F; i += 64) {
+            const int p = i / F;
+            gfeat[b0 * F + i] = pt[p][i - p * F];
+        }
+        wave_fence();
+    }
+    // the wavefronts' sums meet in LDS, one global atomic per weight and block
+#pragma unroll
+    for (int t = 0; t < HT; t++) {
+        const int j = 16 * t + lc;
+#pragma unroll
+        for (int q = 0; q < FT; q++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int i = 16 * q + 4 * lr + r;
+                if (i < F) atomicAdd(&sum[j * FM + i], (double)aw1[q][t][r]);
             }
-            wave_fence();
-        }
-        if (live) {
-#pragma unroll
-            for (int i = 0; i < FM; i++)
-                if (i < F) gfeat[b * F + i] = df[i];
-        }
+        atomicAdd(&sum[PF_HID * FM + j], (double)ab1[t]);
+        atomicAdd(&sum[PF_HID * (FM + 1) + j], (double)aw2[t]);
     }
-    // db2 = sum of g over all points
-    float v = gb2_lane;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    if (lane == 0) atomicAdd(&ab2[0], v);
+    if (lr == 0) atomicAdd(&sum[PF_HID * (FM + 2)], (double)ab2);
     __syncthreads();
-    for (int i = threadIdx.x; i < PF_HID * F; i += PF_BWD_THREADS) atomicAdd(&gW1[i], aW1[i]);
+    for (int i = threadIdx.x; i < PF_HID * F; i += PF_BWD_THREADS)
+        atomicAdd(&gW1[i], (float)sum[(i / F) * FM + i % F]);
     for (int i = threadIdx.x; i < PF_HID; i += PF_BWD_THREADS) {
-        atomicAdd(&gb1[i], ab1[i]);
-        atomicAdd(&gW2[i], aW2[i]);
+        atomicAdd(&gb1[i], (float)sum[PF_HID * FM + i]);
+        atomicAdd(&gW2[i], (float)sum[PF_HID * (FM + 1) + i]);
     }
-    if (threadIdx.x == 0) atomicAdd(&gb2[0], ab2[0]);
+    if (threadIdx.x == 0) atomicAdd(&gb2[0], (float)sum[PF_HID * (FM + 2)]);
 }
 
 #define N3DS_GRID_DISPATCH(KERNEL_LAUNCH)                                                           \
@@ -1640,7 +1714,7 @@ N3DS_EXPORT int n3ds_prop_field_backward(const float* coords, int64_t n_points, 
     const PropArgs P = prop_args(coords, n_points, warp, box_size, embeddings, offsets, num_levels, S, H, gridtype,
                                  align_corners, interp, w1, b1, w2, b2, density_bias);
     int64_t nb;
-    st = prop_blocks(n_points, PF_BWD_THREADS, 3, &nb);  // 3 resident blocks per CU (43 KB of LDS each)
+    st = prop_blocks(n_points, PF_BWD_THREADS, 3, &nb);
     if (st) return st;
     hipStream_t s = (hipStream_t)stream;
 #define LAUNCH_PB(CC, FM, FX)                                                                                    \
