@@ -2324,6 +2324,48 @@ __device__ __forceinline__ void reduce_runs(const RenderArgs& A, const WaveMem& 
     wave_sync();
 }
 
+// The same sums without LDS in between: lanes with the same stroke key are contiguous, so a
+// segmented suffix sum by shuffles (as many steps as the longest run needs) leaves each
+// run's slots with its first lane, which adds them to dst [S, PG].  The LDS transpose above
+// is one chain of LDS and table reads after the other; the shuffles of the slots are
+// independent.  The pair kernel with it: 353 instead of 466 us at 16384 rays x 32 samples of
+// 300 ellipsoids with SH colours, 165 instead of 171 us on the 500-stroke palette.
+template <int NG, typename ACC>
+__device__ __forceinline__ void add_runs(const RenderArgs& A, int lane, int nl, int key, float (&G)[NG], ACC* dst,
+                                         int PG) {
+    const int kprev = __shfl_up(key, 1, 64);
+    const bool head = lane < nl && (lane == 0 || key != kprev);
+    const unsigned long long hm = __ballot(head);
+    const unsigned long long after = hm & ~((2ull << lane) - 1ull);
+    const int end = after ? __builtin_ctzll(after) : nl;
+    for (int off = 1; off < 64; off <<= 1) {
+        const bool in = lane + off < end;
+        if (__ballot(in) == 0ull) break;
+#pragma unroll
+        for (int g = 0; g < NG; g++) {
+            const float u = __shfl_down(G[g], off, 64);
+            if (in) G[g] += u;
+        }
+    }
+    if (!head) return;
+    // slot_column for each slot, the record's fields read once
+    const float* rec = A.table + (int64_t)key * REC;
+    const bool curve = ibits(rec[R_CURVE]) != 0, single = ((uint32_t)ibits(rec[R_FLAGS]) & F_SS) != 0;
+    const int nb = ibits(rec[R_NB]), os = ibits(rec[R_OFFS]), oa = ibits(rec[R_OFFA]), ot = ibits(rec[R_OFFT]);
+    ACC* row = dst + (int64_t)key * PG;
+#pragma unroll
+    for (int g = 0; g < NG; g++) {
+        int col;
+        if (g >= 14) col = A.Pmax + g - 14;
+        else if (curve || g < 2) col = g < nb ? g : -1;
+        else if (g < 5) col = os < 0 || (single && g > 2) ? -1 : os + g - 2;
+        else if (g < 8) col = oa < 0 ? -1 : oa + g - 5;
+        else if (g < 11) col = ot < 0 ? -1 : ot + g - 8;
+        else col = -1;
+        if (col >= 0 && G[g] != 0.f) atomicAdd(row + col, (ACC)G[g]);
+    }
+}
+
 // Pending live pairs of the adjoint, queued per wavefront and class in global memory
 // so that the gradient groups run 64 pairs of one SDF family at a time, across rays.
 // Field-major ring of RCAP slots per class: stroke, ray, sample depth, dL/dalpha,
@@ -2364,8 +2406,6 @@ __device__ __forceinline__ void queued_group(const RenderArgs& A, const WaveMem&
     }
     reduce_runs<NG>(A, w, lane, nl, k, G, dst, PG);
 }
-
-__host__ __device__ constexpr int pairs_wave_floats(int ng) { return 64 * (ng + 1) + 64; }
 
 // Records per page of the split adjoint's pool.  A wavefront starts with one open page per
 // SDF family and takes further ones from a device-wide counter, one returning atomic per
@@ -2418,27 +2458,26 @@ __global__ __launch_bounds__(SCAN_THREADS) void page_scan_kernel(int* __restrict
     }
     if (t == 0) c[n] = carry;
 }
-constexpr int PAIRS_WAVES = 16;  // wavefronts per block of the pair kernel at most (one block per CU)
+constexpr int PAIRS_WAVES = 16;  // wavefronts per block of the pair kernel (one block per CU)
 
 // Split adjoint, second kernel: the records of render_bwd_kernel<MODE 2>, 64 of one SDF
 // family per wavefront, through pair_grad; each stroke's run of lanes is summed into the
-// block's rows (LDS, or the global rows) as in the fused kernel.  When the pool ran out,
-// records of a ray that is flagged for the fused kernel are skipped.
-template <int CID>
-__global__ __launch_bounds__(64 * PAIRS_WAVES) void render_bwd_pairs_kernel(RenderArgs A, float* __restrict__ partials,
-                                                                       int use_lds, float* __restrict__ gdirect) {
-    extern __shared__ float smem[];  // [S * PG] accumulators (use_lds) + per-wavefront regions
+// block's rows in LDS.  When the pool ran out, records of a ray that is flagged for the
+// fused kernel are skipped.
+// ACC: the rows are doubles where they fit the LDS, else floats: 64-bit LDS float atomics
+// run at 2.1 lanes per clock and CU on this card, 32-bit ones at 0.33.
+template <int CID, typename ACC>
+__global__ __launch_bounds__(64 * PAIRS_WAVES) void render_bwd_pairs_kernel(RenderArgs A,
+                                                                            float* __restrict__ partials) {
+    extern __shared__ double rows[];  // [S * PG] of ACC
     constexpr int NG = 15 + num_color_params(CID);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform per wavefront
     const int W = blockDim.x >> 6;
     const int PG = A.Pmax + A.Q + 1;
-    const int64_t nacc = use_lds ? (int64_t)A.S * PG : 0;
-    float* dst = use_lds ? smem : gdirect;
-    for (int64_t i = threadIdx.x; i < nacc; i += blockDim.x) smem[i] = 0.f;
+    const int64_t nacc = (int64_t)A.S * PG;
+    ACC* dst = (ACC*)rows;
+    for (int64_t i = threadIdx.x; i < nacc; i += blockDim.x) dst[i] = (ACC)0;
     __syncthreads();
-    WaveMem w;
-    w.scr = smem + nacc + (int64_t)wave * pairs_wave_floats(NG);
-    w.xo = (int*)(w.scr + 64 * (NG + 1));
     // sp_count holds, after page_scan_kernel, the groups before each page (and the total
     // behind the last); wavefront q takes groups [q G / Q, (q + 1) G / Q)
     const int asked = A.sp_first + *A.sp_next;
@@ -2478,14 +2517,12 @@ __global__ __launch_bounds__(64 * PAIRS_WAVES) void render_bwd_pairs_kernel(Rend
             }
             // empty records only pad a page's last group, so the valid lanes lead it
             const int nl = __popcll(__ballot(k >= 0));
-            reduce_runs<NG>(A, w, lane, nl, k >= 0 ? k : 0x7fffffff, G, dst, PG);
+            add_runs(A, lane, nl, k, G, dst, PG);
         }
     }
-    if (use_lds) {
-        __syncthreads();
-        float* prow = partials + (int64_t)blockIdx.x * nacc;
-        for (int64_t i = threadIdx.x; i < nacc; i += blockDim.x) prow[i] = smem[i];
-    }
+    __syncthreads();
+    float* prow = partials + (int64_t)blockIdx.x * nacc;
+    for (int64_t i = threadIdx.x; i < nacc; i += blockDim.x) prow[i] = (float)dst[i];
 }
 
 // MODE 0: gradient groups window by window; 1: the pending-pair queues (queues !=
@@ -3557,12 +3594,14 @@ N3DS_EXPORT int n3ds_render_forward(const float* origins, const float* direction
 // with their group counts (as many as the workspace given holds, at least min_pages).
 constexpr int SPLIT_WAVES = 4;
 
+typedef void (*PairsKernel)(RenderArgs, float*);
+
 struct SplitPlan {
     bool ok;
     BwdKernel k1, kf;
+    PairsKernel k2;
     int64_t nb1, nb2, nbf;
     int64_t lds1, lds2;
-    int pw;  // wavefronts per block of the pair kernel
     BwdShape bsf;
     int64_t off_rows, off_qf, off_flags, off_pages, min_pages, total;
 };
@@ -3571,12 +3610,13 @@ static int64_t split_page_floats(int64_t pages) {  // group counts (+ total), th
     return (pages + 1 + 63) / 64 * 64 + pages * (RW * SP_PAGE);
 }
 
-typedef void (*PairsKernel)(RenderArgs, float*, int, float*);
-
-static PairsKernel pairs_kernel_ptr(int cid) {
-    static const PairsKernel tab[4] = {render_bwd_pairs_kernel<0>, render_bwd_pairs_kernel<1>,
-                                       render_bwd_pairs_kernel<2>, render_bwd_pairs_kernel<3>};
-    return tab[cid];
+static PairsKernel pairs_kernel_ptr(int cid, bool wide) {
+    static const PairsKernel tab[2][4] = {
+        {render_bwd_pairs_kernel<0, float>, render_bwd_pairs_kernel<1, float>, render_bwd_pairs_kernel<2, float>,
+         render_bwd_pairs_kernel<3, float>},
+        {render_bwd_pairs_kernel<0, double>, render_bwd_pairs_kernel<1, double>, render_bwd_pairs_kernel<2, double>,
+         render_bwd_pairs_kernel<3, double>}};
+    return tab[wide][cid];
 }
 
 static int split_plan(int ns, int cid, int64_t n_rays, int S, int PG, SplitPlan* sp) {
@@ -3587,13 +3627,10 @@ static int split_plan(int ns, int cid, int64_t n_rays, int S, int PG, SplitPlan*
     sp->bsf.use_lds = 0;
     sp->bsf.lds_bytes = (int64_t)BWAVES * bwd_wave_floats(ns, cid) * 4;
     if (sp->bsf.lds_bytes > g_max_lds) return N3DS_OK;
-    const int ng = 15 + num_color_params(cid);
-    // the pair kernel: as many wavefronts per block as the rows leave LDS for
-    sp->pw = 0;
-    for (int wv = PAIRS_WAVES; wv >= 4 && !sp->pw; wv -= 4)
-        if ((int64_t)S * PG * 4 + (int64_t)wv * pairs_wave_floats(ng) * 4 <= g_max_lds) sp->pw = wv;
-    if (!sp->pw) return N3DS_OK;
-    sp->lds2 = (int64_t)S * PG * 4 + (int64_t)sp->pw * pairs_wave_floats(ng) * 4;
+    const bool wide = (int64_t)S * PG * 8 <= g_max_lds;  // rows of doubles in the pair kernel
+    sp->lds2 = (int64_t)S * PG * (wide ? 8 : 4);
+    if (sp->lds2 > g_max_lds) return N3DS_OK;
+    sp->k2 = pairs_kernel_ptr(cid, wide);
     sp->lds1 = (int64_t)SPLIT_WAVES * wave_mem_floats(ns, 5, 3) * 4;
     sp->k1 = bwd_kernel_ptr(ns, cid, 2);
     sp->kf = bwd_kernel_ptr(ns, cid, 1);
@@ -3601,8 +3638,8 @@ static int split_plan(int ns, int cid, int64_t n_rays, int S, int PG, SplitPlan*
         N3DS_HIP_CHECK(hipFuncSetAttribute((const void*)sp->k1, hipFuncAttributeMaxDynamicSharedMemorySize,
                                            (int)sp->lds1));
     if (sp->lds2 > 65536)
-        N3DS_HIP_CHECK(hipFuncSetAttribute((const void*)pairs_kernel_ptr(cid),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)sp->lds2));
+        N3DS_HIP_CHECK(hipFuncSetAttribute((const void*)sp->k2, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           (int)sp->lds2));
     int per_cu = 0;
     N3DS_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)sp->k1, 64 * SPLIT_WAVES,
                                                                 (size_t)sp->lds1));
@@ -3610,8 +3647,8 @@ static int split_plan(int ns, int cid, int64_t n_rays, int S, int PG, SplitPlan*
     const int64_t need1 = (n_rays + SPLIT_WAVES - 1) / SPLIT_WAVES;
     if (sp->nb1 > need1) sp->nb1 = need1;
     per_cu = 0;
-    N3DS_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)pairs_kernel_ptr(cid),
-                                                                64 * sp->pw, (size_t)sp->lds2));
+    N3DS_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)sp->k2, 64 * PAIRS_WAVES,
+                                                                (size_t)sp->lds2));
     sp->nb2 = (int64_t)g_num_cu * (per_cu < 1 ? 1 : per_cu);
     if (bwd_blocks(sp->kf, sp->bsf, n_rays, &sp->nbf)) return -1;
     const int64_t tot = (int64_t)S * PG;
@@ -3736,8 +3773,7 @@ static int render_backward_impl(const float* origins, const float* directions, c
             hipLaunchKernelGGL(page_scan_kernel, dim3(1), dim3(SCAN_THREADS), 0, s, A.sp_count, A.sp_next, A.sp_first, A.sp_pages,
                                rows + sp.nb2 * tot, tot);
             N3DS_LAUNCH_CHECK();
-            hipLaunchKernelGGL(pairs_kernel_ptr(color_id), dim3((unsigned)sp.nb2), dim3(64 * sp.pw), (size_t)sp.lds2,
-                               s, A, rows, 1, (float*)nullptr);
+            hipLaunchKernelGGL(sp.k2, dim3((unsigned)sp.nb2), dim3(64 * PAIRS_WAVES), (size_t)sp.lds2, s, A, rows);
             N3DS_LAUNCH_CHECK();
             hipLaunchKernelGGL(sp.kf, dim3((unsigned)sp.nbf), dim3(64 * sp.bsf.waves), (size_t)sp.bsf.lds_bytes, s, A,
                                grad_rgb, grad_acc, grad_depth, state, (float*)nullptr, 0, rows + sp.nb2 * tot,
