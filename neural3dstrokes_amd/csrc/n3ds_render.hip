@@ -36,6 +36,8 @@
 #include <algorithm>
 #include <mutex>
 
+#include <type_traits>
+
 #include "n3ds_capi.h"
 #include "n3ds_stroke_common.h"
 
@@ -598,6 +600,10 @@ struct WaveMem {
 __host__ __device__ constexpr int wave_mem_floats(int ns, int npf, int ng) {
     return 64 * ns + 5 * HMAX + 128 + npf * PBUF + (ng > 0 ? 64 * (ng + 1) + PBUF : 0);
 }
+
+// MODE 2 of render_bwd_kernel: 16-bit live-pair codes in place of the gradient slots, and
+// 16-bit lists
+__host__ __device__ constexpr int split_wave_floats(int ns) { return 64 * ns + 5 * HMAX + 128 + 5 * PBUF + PBUF; }
 
 __device__ __forceinline__ WaveMem wave_mem(float* base, int ns, int npf, int ng = 0) {
     WaveMem w;
@@ -2543,7 +2549,13 @@ __global__ __launch_bounds__(64 * BWAVES) void render_bwd_kernel(RenderArgs A0, 
     constexpr bool QUEUE = MODE != 0;
     constexpr int NQ = num_color_params(CID);
     constexpr int NG = 15 + NQ;  // gradient slots per pair
-    constexpr int NGL = MODE == 2 ? 3 : NG;  // LDS slots per lane (MODE 2: the live-pair codes only)
+    // live-pair codes (hit << 2 | class) and lists (hit << SH | pair); MODE 2 has them in 16
+    // bits and no gradient slots, which leaves room for four of its blocks on a CU instead of
+    // three (278 instead of 343 us on the 500-stroke palette, 65536 rays x 128 samples)
+    typedef typename std::conditional<MODE == 2, short, int>::type Code;
+    typedef typename std::conditional<MODE == 2, unsigned short, int>::type Live;
+    constexpr int SH = MODE == 2 ? 8 : 16, PMASK = (1 << SH) - 1;
+    static_assert(PBUF <= 1 << 8 && HMAX <= 1 << 7, "a hit and a pair fit 16 bits");
     constexpr int NPF = 5;       // per-pair values: alpha -> dL/dalpha, colour / dL/d(density, colour)
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform per wavefront
     const int W = blockDim.x >> 6;
@@ -2573,7 +2585,9 @@ __global__ __launch_bounds__(64 * BWAVES) void render_bwd_kernel(RenderArgs A0, 
     float* gacc = smem;
     for (int64_t i = threadIdx.x; i < nacc; i += blockDim.x) gacc[i] = 0.f;
     __syncthreads();
-    const WaveMem w = wave_mem(smem + nacc_max + wave * wave_mem_floats(NS, NPF, NGL), NS, NPF, NGL);
+    const int wfloats = MODE == 2 ? split_wave_floats(NS) : wave_mem_floats(NS, NPF, NG);
+    const WaveMem w = wave_mem(smem + nacc_max + wave * wfloats, NS, NPF, MODE == 2 ? 1 : NG);
+    Live* const ul = (Live*)w.ul;
     const int64_t N = A.R * (int64_t)A.n;
     // MODE 2: this wavefront's open pages and how many records each holds
     const int own = NCLASS * (int)(blockIdx.x * W + wave);
@@ -2898,8 +2912,8 @@ __global__ __launch_bounds__(64 * BWAVES) void render_bwd_kernel(RenderArgs A0, 
                 // (3) parameter gradients per pair, reduced per stroke.  Only pairs with a
                 //     nonzero adjoint contribute (alpha = 0 pairs do not): compact them first,
                 //     in order, so that each stroke's pairs stay contiguous
-                //     class by class (w.ul: class segments of (hit << 16 | pair), each in pair order)
-                int* code = (int*)w.scr;  // [wp] hit << 2 | class of a live pair, -1 otherwise
+                //     class by class (ul: class segments of (hit << SH | pair), each in pair order)
+                Code* code = (Code*)w.scr;  // [wp] hit << 2 | class of a live pair, -1 otherwise
                 int xn[NCLASS] = {0, 0, 0};
                 for (int p0 = 0; p0 < wp; p0 += 64) {
                     const int p = p0 + lane;
@@ -2911,7 +2925,7 @@ __global__ __launch_bounds__(64 * BWAVES) void render_bwd_kernel(RenderArgs A0, 
                         const int c = find_hit(w, c0, c1, wbase, p);
                         cd = (c << 2) | (w.ccls[c] & 3);
                     }
-                    if (p < wp) code[p] = cd;
+                    if (p < wp) code[p] = (Code)cd;
 #pragma unroll
                     for (int xc = 0; xc < NCLASS; xc++) xn[xc] += __popcll(__ballot(cd >= 0 && (cd & 3) == xc));
                 }
@@ -2929,7 +2943,7 @@ __global__ __launch_bounds__(64 * BWAVES) void render_bwd_kernel(RenderArgs A0, 
                         for (int xc = 0; xc < NCLASS; xc++) {
                             const bool in = cd >= 0 && (cd & 3) == xc;
                             const unsigned long long m = __ballot(in);
-                            if (in) w.ul[xf[xc] + __popcll(m & ((1ull << lane) - 1ull))] = ((cd >> 2) << 16) | p;
+                            if (in) ul[xf[xc] + __popcll(m & ((1ull << lane) - 1ull))] = (Live)(((cd >> 2) << SH) | p);
                             xf[xc] += __popcll(m);
                         }
                     }
@@ -2954,8 +2968,8 @@ __global__ __launch_bounds__(64 * BWAVES) void render_bwd_kernel(RenderArgs A0, 
                             }
                         }
                         for (int u = lane; u < nx; u += 64) {
-                            const int e = w.ul[xs[xc] + u];
-                            const int p = e & 0xffff, c = e >> 16;
+                            const int e = ul[xs[xc] + u];
+                            const int p = e & PMASK, c = e >> SH;
                             const int slot = cur[xc] + u;
                             float* L = A.sp_list + (int64_t)(slot < SP_PAGE ? page[xc] : fresh) * (RW * SP_PAGE) +
                                        slot % SP_PAGE;
@@ -2988,8 +3002,8 @@ __global__ __launch_bounds__(64 * BWAVES) void render_bwd_kernel(RenderArgs A0, 
                         const int nx = xs[xc + 1] - xs[xc];
                         float* rq = queue + xc * (RCAP * RW);
                         for (int u = lane; u < nx; u += 64) {
-                            const int e = w.ul[xs[xc] + u];
-                            const int p = e & 0xffff, c = e >> 16;
+                            const int e = ul[xs[xc] + u];
+                            const int p = e & PMASK, c = e >> SH;
                             const int slot = (qtail[xc] + u) % RCAP;
                             rq[slot] = __int_as_float(w.ck[c]);
                             rq[RCAP + slot] = __int_as_float((int)ray);
@@ -3015,8 +3029,8 @@ __global__ __launch_bounds__(64 * BWAVES) void render_bwd_kernel(RenderArgs A0, 
                         for (int g = 0; g < NG; g++) G[g] = 0.f;
                         int c = 0x7fffffff;  // sorts after every hit index
                         if (u < nu) {
-                            const int p = w.ul[u] & 0xffff;
-                            c = w.ul[u] >> 16;
+                            const int p = ul[u] & PMASK;
+                            c = ul[u] >> SH;
                             const float ga = w.pb[p];
                             const float gdw = w.pb[PBUF + p];
                             const V3 gcol = v3(w.pb[2 * PBUF + p], w.pb[3 * PBUF + p], w.pb[4 * PBUF + p]);
@@ -3631,7 +3645,7 @@ static int split_plan(int ns, int cid, int64_t n_rays, int S, int PG, SplitPlan*
     sp->lds2 = (int64_t)S * PG * (wide ? 8 : 4);
     if (sp->lds2 > g_max_lds) return N3DS_OK;
     sp->k2 = pairs_kernel_ptr(cid, wide);
-    sp->lds1 = (int64_t)SPLIT_WAVES * wave_mem_floats(ns, 5, 3) * 4;
+    sp->lds1 = (int64_t)SPLIT_WAVES * split_wave_floats(ns) * 4;
     sp->k1 = bwd_kernel_ptr(ns, cid, 2);
     sp->kf = bwd_kernel_ptr(ns, cid, 1);
     if (sp->lds1 > 65536)
