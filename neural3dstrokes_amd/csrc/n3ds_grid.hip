@@ -10,6 +10,8 @@
 // Index math is uint32 with wrap-around exactly as gridencoder.cu:50-84.
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
+
 #include "n3ds_capi.h"
 
 namespace n3ds {
@@ -1151,7 +1153,9 @@ static int gs_launch(const T* grad, const float* inputs, const int* offsets, int
 constexpr int PF_HID = 64;
 constexpr int PF_MAXF = 32;
 constexpr int PF_FWD_THREADS = 256;
-constexpr int PF_BWD_THREADS = 256;
+// Adjoint: one block per CU while its registers allow 12 wavefronts (450 instead of 606 us at
+// 4.2 M points and 10 features; a third of the atomic additions at the end), else three.
+constexpr int pf_bwd_threads(int fm) { return fm <= 12 ? 768 : 256; }
 
 struct PropArgs {
     const float* coords;  // [N, 3] sample positions
@@ -1204,6 +1208,212 @@ __device__ __forceinline__ void prop_features(const PropArgs& P, const float* x0
     }
 }
 
+// Features of many points with the levels in step over the whole chip, for tables larger than
+// an XCD's L2.  One resident block per CU owns a run of points, kept in LDS, and all blocks
+// walk the levels at the same pace, a hashed level's table in parts of at most an L2: what is
+// gathered from at one time stays in every L2.  Blocks at any level of their own hold several
+// levels' tables at once, and most gathers go to memory, which answers 55 G scattered lines a
+// second here (4.2 M points, 10 levels of up to 8 MB: 1843 us, 108 M lines).  Gathers that hit
+// the L2 are then bound by the vector cache, 2 to 3 clocks a line: a load of 16 bytes serves
+// both corners of most x edges.  The rows of a point's corners wait in registers until the last
+// part, so that they are summed in the one kernel's order, to the bit (a hidden unit at its
+// kink passes on or not by the last bit of its features).  Features are written level by
+// level, [L, n, C]; with the head after it 1435 us (1538 + 140 with whole levels of 8 MB, 1149 +
+// 140 with sums kept from part to part).
+constexpr int LS_THREADS = 1024;
+constexpr int LS_POINTS = 8;                // per thread and round at most
+constexpr int64_t LS_PART_BYTES = 4 << 20;  // of a level's table gathered from at one time
+
+// A table row of 2 or 4 bytes as it is held until the sum
+template <typename T, int C>
+union GridRow {
+    uint32_t bits;
+    T v[C];
+};
+
+struct LevelPoint {
+    float f[3];
+    uint32_t pg[3];
+    bool oob;
+};
+
+// as level_coords
+__device__ __forceinline__ LevelPoint level_point(const float* x, float scale, int align, int interp) {
+    LevelPoint p;
+    p.oob = false;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const float xd = x[d * LS_THREADS];
+        if (xd < 0.f || xd > 1.f) p.oob = true;
+        float t = fmaf(xd, scale, align ? 0.0f : 0.5f);
+        const float fl = floorf(t);
+        p.pg[d] = (uint32_t)fl;
+        t -= fl;
+        if (interp == 1) t = t * t * (3.f - 2.f * t);
+        p.f[d] = t;
+    }
+    return p;
+}
+
+template <typename T, int C>
+__device__ __forceinline__ void level_sum(const LevelPoint& p, const GridRow<T, C> (&row)[8], float (&acc)[C]) {
+#pragma unroll
+    for (int c = 0; c < C; c++) acc[c] = 0.f;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        float w = 1.f;
+#pragma unroll
+        for (int d = 0; d < 3; d++) w *= k & (1 << d) ? p.f[d] : 1.f - p.f[d];
+#pragma unroll
+        for (int c = 0; c < C; c++) acc[c] += w * to_f<T>(row[k].v[c]);
+    }
+    if (p.oob)
+#pragma unroll
+        for (int c = 0; c < C; c++) acc[c] = 0.f;
+}
+
+// row r mod QR of the QR rows in 16 bytes (a row of 2 bytes in the low half)
+template <int QR>
+__device__ __forceinline__ uint32_t quad_row(uint4 e, uint32_t r) {
+    const uint32_t i = QR == 8 ? r >> 1 : r;
+    const uint32_t lo = i & 1 ? e.y : e.x, hi = i & 1 ? e.w : e.z;
+    const uint32_t w = i & 2 ? hi : lo;
+    return QR == 8 && (r & 1) ? w >> 16 : w;
+}
+
+// The corners of a level hashed into hs = 2^k rows that lie in [lo, lo + width), a multiple of
+// 16 rows; the others' rows stay as they are.
+template <typename T, int C>
+__device__ __forceinline__ void level_hashed(const LevelPoint& p, const T* __restrict__ g, uint32_t hs, uint32_t lo,
+                                             uint32_t width, GridRow<T, C> (&row)[8]) {
+    constexpr int QR = 16 / (C * (int)sizeof(T));  // rows of 16 bytes
+    static_assert(QR == 4 || QR == 8, "rows of 2 or 4 bytes");
+    const uint32_t y0 = p.pg[1] * 2654435761u, y1 = y0 + 2654435761u;
+    const uint32_t z0 = p.pg[2] * 805459861u, z1 = z0 + 805459861u;
+#pragma unroll
+    for (int k = 0; k < 8; k += 2) {
+        // the two corners of an x edge: x and x + 1 mostly differ in the low bits only
+        const uint32_t yz = (k & 2 ? y1 : y0) ^ (k & 4 ? z1 : z0);
+        const uint32_t a = (p.pg[0] ^ yz) & (hs - 1), b = ((p.pg[0] + 1) ^ yz) & (hs - 1);
+        const bool ina = !p.oob && a - lo < width, inb = !p.oob && b - lo < width;
+        union {
+            uint4 q;
+            T v[QR * C];
+        } e;  // not used unless loaded
+        if (ina) e.q = *(const uint4*)(g + (a & ~(uint32_t)(QR - 1)) * C);
+        if constexpr (sizeof(T) == 4) {
+            T va = e.v[0], vb = e.v[0];
+#pragma unroll
+            for (int i = 1; i < 4; i++) {
+                va = (a & 3) == i ? e.v[i] : va;
+                vb = (b & 3) == i ? e.v[i] : vb;
+            }
+            row[k].v[0] = ina ? va : row[k].v[0];
+            row[k + 1].v[0] = ina && (a ^ b) < QR ? vb : row[k + 1].v[0];
+        } else {
+            const uint32_t va = quad_row<QR>(e.q, a), vb = quad_row<QR>(e.q, b);
+            row[k].bits = ina ? va : row[k].bits;
+            row[k + 1].bits = ina && (a ^ b) < QR ? vb : row[k + 1].bits;
+        }
+        if (inb && (a ^ b) >= QR) {
+#pragma unroll
+            for (int c = 0; c < C; c++) row[k + 1].v[c] = g[b * C + c];
+        }
+    }
+}
+
+// any other level; r1 > 0: a lattice of r1^3 <= hs rows (no remainder to take)
+template <typename T, int C>
+__device__ __forceinline__ void level_direct(const LevelPoint& p, const T* __restrict__ g, uint32_t hs, uint32_t res,
+                                             uint32_t r1, int gridtype, int align, GridRow<T, C> (&row)[8]) {
+    if (p.oob) return;
+    const uint32_t r0 = p.pg[0] + r1 * (p.pg[1] + r1 * p.pg[2]);
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        uint32_t at = r0 + (k & 1) + (k & 2 ? r1 : 0) + (k & 4 ? r1 * r1 : 0);
+        if (r1 == 0) {
+            const uint32_t loc[3] = {p.pg[0] + (k & 1), p.pg[1] + ((k >> 1) & 1), p.pg[2] + (k >> 2)};
+            at = grid_index<3>(gridtype, align != 0, hs, res, loc);
+        }
+#pragma unroll
+        for (int c = 0; c < C; c++) row[k].v[c] = g[at * C + c];
+    }
+}
+
+template <typename T, int C>
+__device__ __forceinline__ void level_store(float* __restrict__ stage, int64_t n, int level, int64_t b,
+                                            const float (&acc)[C]) {
+    if (b < n) {
+#pragma unroll
+        for (int c = 0; c < C; c++) stage[((int64_t)level * n + b) * C + c] = acc[c];
+    }
+}
+
+template <typename T, int C>
+__global__ __launch_bounds__(LS_THREADS) void prop_level_kernel(PropArgs P, int64_t b0, int64_t n,
+                                                                float* __restrict__ stage, int ppt) {
+    extern __shared__ float ls[];  // [ppt][3][LS_THREADS]: the points' coordinates
+    const int t = threadIdx.x;
+    for (int64_t p0 = (int64_t)blockIdx.x * LS_THREADS * ppt; p0 < n; p0 += (int64_t)gridDim.x * LS_THREADS * ppt) {
+        for (int q = 0; q < ppt; q++) {
+            float cw[3], x01[3];
+            prop_warp(P, b0 + min(p0 + q * LS_THREADS + t, n - 1), cw, x01);
+#pragma unroll
+            for (int d = 0; d < 3; d++) ls[(q * 3 + d) * LS_THREADS + t] = x01[d];
+        }
+        for (int level = 0; level < P.L; level++) {
+            const uint32_t hs = (uint32_t)(P.offsets[level + 1] - P.offsets[level]);
+            const float scale = P.lt.scale[level];
+            const uint32_t res = (uint32_t)ceilf(scale) + 1, r1 = res + 1;
+            const T* g = (const T*)P.emb + (int64_t)P.offsets[level] * C;
+            // r1 below 1626: its cube fits 32 bits; below 65536: its square does
+            const bool lattice = !P.align && r1 < 1626u && r1 * r1 * r1 <= hs;
+            const bool hashed = !P.align && P.gridtype == 0 && r1 < 65536u && !lattice && (hs & (hs - 1)) == 0 &&
+                                !(r1 >= 1626u && r1 * r1 <= hs) && hs >= 16 && ((uintptr_t)g & 15) == 0;
+            const uint32_t part = (uint32_t)(LS_PART_BYTES / (C * (int)sizeof(T)));
+            if (hashed && hs > part) {
+                GridRow<T, C> row[LS_POINTS][8];
+#pragma unroll
+                for (int q = 0; q < LS_POINTS; q++)
+#pragma unroll
+                    for (int k = 0; k < 8; k++) row[q][k].bits = 0;
+                for (uint32_t lo = 0; lo < hs; lo += part) {
+#pragma unroll
+                    for (int q = 0; q < LS_POINTS; q++) {
+                        if (q < ppt)
+                            level_hashed<T, C>(level_point(ls + q * 3 * LS_THREADS + t, scale, 0, 0), g, hs, lo, part,
+                                               row[q]);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+#pragma unroll
+                for (int q = 0; q < LS_POINTS; q++) {
+                    if (q < ppt) {
+                        float acc[C];
+                        level_sum<T, C>(level_point(ls + q * 3 * LS_THREADS + t, scale, 0, P.interp), row[q], acc);
+                        level_store<T, C>(stage, n, level, p0 + q * LS_THREADS + t, acc);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            } else {
+#pragma unroll 2
+                for (int q = 0; q < ppt; q++) {
+                    LevelPoint p = level_point(ls + q * 3 * LS_THREADS + t, scale, P.align, P.interp);
+                    if (hs == 0) p.oob = true;  // an empty level
+                    GridRow<T, C> row[8];
+#pragma unroll
+                    for (int k = 0; k < 8; k++) row[k].bits = 0;
+                    if (hashed) level_hashed<T, C>(p, g, hs, 0, hs, row);
+                    else level_direct<T, C>(p, g, hs, res, lattice ? r1 : 0, P.gridtype, P.align, row);
+                    float acc[C];
+                    level_sum<T, C>(p, row, acc);
+                    level_store<T, C>(stage, n, level, p0 + q * LS_THREADS + t, acc);
+                }
+            }
+        }
+    }
+}
+
 // torch.nn.functional.softplus (beta 1, threshold 20) and its derivative
 __device__ __forceinline__ float softplus20(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 __device__ __forceinline__ float dsoftplus20(float x) { return x > 20.f ? 1.f : 1.f / (1.f + expf(-x)); }
@@ -1225,8 +1435,10 @@ __device__ __forceinline__ float prop_raw(const float* sW1, const float* sb1, co
 
 // FM: per-lane feature capacity (16 or 32 >= F)
 // FX > 0: the feature count is FX (= FM) at compile time
-template <typename T, int C, int FM, int FX = 0>
-__global__ __launch_bounds__(PF_FWD_THREADS) void prop_fwd_kernel(PropArgs P, float* __restrict__ density,
+// STAGED: points [b0, b0 + n) with their features from prop_level_kernel's [L, n, C]
+template <typename T, int C, int FM, int FX = 0, bool STAGED = false>
+__global__ __launch_bounds__(PF_FWD_THREADS) void prop_fwd_kernel(PropArgs P, const float* __restrict__ stage,
+                                                                  int64_t b0, int64_t n, float* __restrict__ density,
                                                                   float* __restrict__ coord_out,
                                                                   float* __restrict__ feat_out,
                                                                   float* __restrict__ x01_out) {
@@ -1239,11 +1451,19 @@ __global__ __launch_bounds__(PF_FWD_THREADS) void prop_fwd_kernel(PropArgs P, fl
     }
     __syncthreads();
     const float b2 = P.b2[0];
-    for (int64_t b = (int64_t)blockIdx.x * PF_FWD_THREADS + threadIdx.x; b < P.N;
-         b += (int64_t)gridDim.x * PF_FWD_THREADS) {
+    for (int64_t i = (int64_t)blockIdx.x * PF_FWD_THREADS + threadIdx.x; i < n;
+         i += (int64_t)gridDim.x * PF_FWD_THREADS) {
+        const int64_t b = b0 + i;
         float cw[3], x01[3], f[FM];
         prop_warp(P, b, cw, x01);
-        prop_features<T, C, FM>(P, x01, f);
+        if constexpr (STAGED) {
+#pragma unroll
+            for (int l = 0; l < FM / C; l++)
+#pragma unroll
+                for (int c = 0; c < C; c++) f[l * C + c] = l < P.L ? stage[((int64_t)l * n + i) * C + c] : 0.f;
+        } else {
+            prop_features<T, C, FM>(P, x01, f);
+        }
         const float raw = prop_raw<FM>(sW1, sb1, sW2, b2, F, f);
         density[b] = softplus20(raw + P.dbias);
         if (coord_out) {
@@ -1282,19 +1502,19 @@ __device__ __forceinline__ f4 mfma16(float a, float b, f4 c) {
 // 56 matrix instructions per 16 points and 10 features.  The vector version went through
 // LDS for every product (7 LDS reads per point and hidden unit): 1560 us at 4.2 M points.
 template <typename T, int C, int FM, int FX = 0>
-__global__ __launch_bounds__(PF_BWD_THREADS) void prop_bwd_kernel(PropArgs P, const float* __restrict__ gdens,
+__global__ __launch_bounds__(pf_bwd_threads(FM)) void prop_bwd_kernel(PropArgs P, const float* __restrict__ gdens,
                                                                   const float* __restrict__ feat_in,
                                                                   float* __restrict__ gfeat, float* __restrict__ x01_out,
                                                                   float* __restrict__ gW1, float* __restrict__ gb1,
                                                                   float* __restrict__ gW2, float* __restrict__ gb2) {
-    constexpr int NW = PF_BWD_THREADS / 64, KS = (FM + 3) / 4, FT = (FM + 15) / 16, HT = PF_HID / 16;
+    constexpr int NT = pf_bwd_threads(FM), NW = NT / 64, KS = (FM + 3) / 4, FT = (FM + 15) / 16, HT = PF_HID / 16;
     constexpr int FP = 16 * FT + 1;  // row of a point's features in LDS
     __shared__ float sf[NW][64][FP];  // a wavefront's 64 points: features, then their gradients
     __shared__ double sum[PF_HID * (FM + 2) + 1];  // dW1 [hidden, feature], db1, dW2, db2 of the block
     const int F = FX > 0 ? FX : P.L * C;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform per wavefront
     const int lc = lane & 15, lr = lane >> 4;
-    for (int i = threadIdx.x; i < PF_HID * (FM + 2) + 1; i += PF_BWD_THREADS) sum[i] = 0.0;
+    for (int i = threadIdx.x; i < PF_HID * (FM + 2) + 1; i += NT) sum[i] = 0.0;
     // constant operands: w1[t][k] = W1[16 t + lc][4 k + lr], w1t[q][t][r] = W1[16 t + 4 lr + r][16 q + lc]
     float w1[HT][KS], w1t[FT][HT][4], b1q[HT], w2q[HT];
     f4 b1p[HT], w2p[HT];
@@ -1434,9 +1654,9 @@ __global__ __launch_bounds__(PF_BWD_THREADS) void prop_bwd_kernel(PropArgs P, co
     }
     if (lr == 0) atomicAdd(&sum[PF_HID * (FM + 2)], (double)ab2);
     __syncthreads();
-    for (int i = threadIdx.x; i < PF_HID * F; i += PF_BWD_THREADS)
+    for (int i = threadIdx.x; i < PF_HID * F; i += NT)
         atomicAdd(&gW1[i], (float)sum[(i / F) * FM + i % F]);
-    for (int i = threadIdx.x; i < PF_HID; i += PF_BWD_THREADS) {
+    for (int i = threadIdx.x; i < PF_HID; i += NT) {
         atomicAdd(&gb1[i], (float)sum[PF_HID * FM + i]);
         atomicAdd(&gW2[i], (float)sum[PF_HID * (FM + 1) + i]);
     }
@@ -1658,13 +1878,36 @@ static PropArgs prop_args(const float* coords, int64_t N, int warp, float box_si
     return P;
 }
 
-N3DS_EXPORT int n3ds_prop_field_forward(const float* coords, int64_t n_points, int warp, float box_size,
-                                        const void* embeddings, const int32_t* offsets, int num_levels,
-                                        int level_dim, float S, int H, int gridtype, int align_corners, int interp,
-                                        int dtype, const float* w1, const float* b1, const float* w2,
-                                        const float* b2, float density_bias, float* density_out,
-                                        float* coord_out, float* features_out, float* grid_inputs_out,
-                                        void* stream) {
+// The staged features pay where the tables do not fit an L2, 16 bytes hold four rows or more,
+// and there are enough points to fetch every table into every L2 for.  Forward with kept
+// features, staged against fused (us), 10 levels:
+//   rows of 4 bytes, tables of 57 MB: 2^17 points 75 / 65, 2^18 97 / 122, 2^22 1435 / 1848;
+//   15 MB: 2^17 65 / 47, 2^18 72 / 88, 2^22 970 / 1420; 4.2 MB: 2^18 62 / 63, 2^21 385 / 437;
+//   two half features, levels of 2 MB: 2^17 73 / 50, 2^18 89 / 93, 2^22 1130 / 1478; of 8 MB:
+//   2^18 244 / 126, 2^21 1092 / 930;
+//   rows of 8 bytes, 30 MB: 2^18 117 / 110, 2^21 917 / 862; of 16 bytes: 2^21 1412 / 1119.
+constexpr int64_t PF_STAGE_TABLE = 4 << 20;  // bytes of all tables
+constexpr int64_t PF_STAGE_ROW = 4;          // bytes of a row at most
+constexpr int64_t PF_STAGE_POINTS = 1 << 18;
+constexpr int64_t PF_STAGE_CHUNK = 1 << 22;  // points whose features are staged at one time
+
+N3DS_EXPORT int64_t n3ds_prop_field_workspace_bytes(int64_t n_points, int num_levels, int level_dim, int64_t n_rows,
+                                                    int dtype) {
+    if (n_points < PF_STAGE_POINTS || num_levels < 1 || level_dim < 1 || n_rows < 0) return 0;
+    const int64_t row = level_dim * (dtype == 1 ? 2 : 4);
+    if (row > PF_STAGE_ROW || n_rows * row <= PF_STAGE_TABLE) return 0;
+    // two half features in parts of a level: the rows kept do not fit the registers
+    if (level_dim == 2 && n_rows * row > num_levels * LS_PART_BYTES) return 0;
+    return std::min(n_points, PF_STAGE_CHUNK) * num_levels * level_dim * 4;
+}
+
+N3DS_EXPORT int n3ds_prop_field_forward_ws(const float* coords, int64_t n_points, int warp, float box_size,
+                                           const void* embeddings, const int32_t* offsets, int num_levels,
+                                           int level_dim, float S, int H, int gridtype, int align_corners, int interp,
+                                           int dtype, const float* w1, const float* b1, const float* w2,
+                                           const float* b2, float density_bias, float* density_out,
+                                           float* coord_out, float* features_out, float* grid_inputs_out,
+                                           int64_t n_rows, void* workspace, int64_t workspace_bytes, void* stream) {
     N3DS_REQUIRE((features_out == nullptr) == (grid_inputs_out == nullptr),
                  "features_out and grid_inputs_out are kept together");
     int st = prop_check(n_points, level_dim, num_levels, dtype, warp);
@@ -1672,32 +1915,76 @@ N3DS_EXPORT int n3ds_prop_field_forward(const float* coords, int64_t n_points, i
     if (n_points == 0) return N3DS_OK;
     const PropArgs P = prop_args(coords, n_points, warp, box_size, embeddings, offsets, num_levels, S, H, gridtype,
                                  align_corners, interp, w1, b1, w2, b2, density_bias);
-    int64_t nb;
-    st = prop_blocks(n_points, PF_FWD_THREADS, 8, &nb);
-    if (st) return st;
     hipStream_t s = (hipStream_t)stream;
+    const int64_t need = n3ds_prop_field_workspace_bytes(n_points, num_levels, level_dim, n_rows, dtype);
+    const bool staged = need > 0 && workspace != nullptr && workspace_bytes >= need;
+    float* stage = (float*)workspace;
+    const int64_t step = staged ? PF_STAGE_CHUNK : n_points;
+    for (int64_t at = 0; at < n_points; at += step) {
+        const int64_t n = std::min(step, n_points - at);
+        int64_t nb;
+        if (staged) {
+            // one block per CU; its points in as few equal rounds as the registers allow
+            const int cap = LS_POINTS;
+            st = prop_blocks(n, LS_THREADS, 1, &nb);
+            if (st) return st;
+            const int64_t per = (n + nb * LS_THREADS - 1) / (nb * LS_THREADS), rounds = (per + cap - 1) / cap;
+            const int ppt = (int)((per + rounds - 1) / rounds);
+            const size_t lds = (size_t)ppt * 3 * LS_THREADS * 4;
+#define LAUNCH_PL(T, CC)                                                                                         \
+    {                                                                                                            \
+        N3DS_HIP_CHECK(hipFuncSetAttribute((const void*)prop_level_kernel<T, CC>,                                \
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, LS_POINTS * 3 * LS_THREADS * 4)); \
+        hipLaunchKernelGGL((prop_level_kernel<T, CC>), dim3((unsigned)nb), dim3(LS_THREADS), lds, s, P, at, n,   \
+                           stage, ppt);                                                                          \
+    }
+            if (dtype == 0) LAUNCH_PL(float, 1)
+            else if (level_dim == 1) LAUNCH_PL(__half, 1)
+            else LAUNCH_PL(__half, 2)
+#undef LAUNCH_PL
+            N3DS_LAUNCH_CHECK();
+        }
+        st = prop_blocks(n, PF_FWD_THREADS, 8, &nb);
+        if (st) return st;
 #define LAUNCH_PF(CC, FM, FX)                                                                                    \
-    if (dtype == 0)                                                                                              \
+    if (CC <= 2 && staged)                                                                                       \
+        hipLaunchKernelGGL((prop_fwd_kernel<float, CC <= 2 ? CC : 1, FM, FX, true>), dim3((unsigned)nb),         \
+                           dim3(PF_FWD_THREADS), 0, s, P, stage, at, n, density_out, coord_out, features_out,    \
+                           grid_inputs_out);                                                                     \
+    else if (dtype == 0)                                                                                         \
         hipLaunchKernelGGL((prop_fwd_kernel<float, CC, FM, FX>), dim3((unsigned)nb), dim3(PF_FWD_THREADS), 0, s, \
-                           P, density_out, coord_out, features_out, grid_inputs_out);                            \
+                           P, stage, at, n, density_out, coord_out, features_out, grid_inputs_out);              \
     else                                                                                                         \
         hipLaunchKernelGGL((prop_fwd_kernel<__half, CC, FM, FX>), dim3((unsigned)nb), dim3(PF_FWD_THREADS), 0,   \
-                           s, P, density_out, coord_out, features_out, grid_inputs_out);
-    const bool small = num_levels * level_dim <= 16;
-    if (level_dim == 1 && num_levels == 10) {
-        LAUNCH_PF(1, 10, 10)
-    } else if (level_dim == 2 && num_levels == 10) {
-        LAUNCH_PF(2, 20, 20)
-    } else if (level_dim == 1) {
-        if (small) { LAUNCH_PF(1, 16, 0) } else { LAUNCH_PF(1, 32, 0) }
-    } else if (level_dim == 2) {
-        if (small) { LAUNCH_PF(2, 16, 0) } else { LAUNCH_PF(2, 32, 0) }
-    } else {
-        if (small) { LAUNCH_PF(4, 16, 0) } else { LAUNCH_PF(4, 32, 0) }
-    }
+                           s, P, stage, at, n, density_out, coord_out, features_out, grid_inputs_out);
+        const bool small = num_levels * level_dim <= 16;
+        if (level_dim == 1 && num_levels == 10) {
+            LAUNCH_PF(1, 10, 10)
+        } else if (level_dim == 2 && num_levels == 10) {
+            LAUNCH_PF(2, 20, 20)
+        } else if (level_dim == 1) {
+            if (small) { LAUNCH_PF(1, 16, 0) } else { LAUNCH_PF(1, 32, 0) }
+        } else if (level_dim == 2) {
+            if (small) { LAUNCH_PF(2, 16, 0) } else { LAUNCH_PF(2, 32, 0) }
+        } else {
+            if (small) { LAUNCH_PF(4, 16, 0) } else { LAUNCH_PF(4, 32, 0) }
+        }
 #undef LAUNCH_PF
-    N3DS_LAUNCH_CHECK();
+        N3DS_LAUNCH_CHECK();
+    }
     return N3DS_OK;
+}
+
+N3DS_EXPORT int n3ds_prop_field_forward(const float* coords, int64_t n_points, int warp, float box_size,
+                                        const void* embeddings, const int32_t* offsets, int num_levels,
+                                        int level_dim, float S, int H, int gridtype, int align_corners, int interp,
+                                        int dtype, const float* w1, const float* b1, const float* w2,
+                                        const float* b2, float density_bias, float* density_out,
+                                        float* coord_out, float* features_out, float* grid_inputs_out,
+                                        void* stream) {
+    return n3ds_prop_field_forward_ws(coords, n_points, warp, box_size, embeddings, offsets, num_levels, level_dim, S,
+                                      H, gridtype, align_corners, interp, dtype, w1, b1, w2, b2, density_bias,
+                                      density_out, coord_out, features_out, grid_inputs_out, 0, nullptr, 0, stream);
 }
 
 N3DS_EXPORT int n3ds_prop_field_backward(const float* coords, int64_t n_points, int warp, float box_size,
@@ -1714,16 +2001,16 @@ N3DS_EXPORT int n3ds_prop_field_backward(const float* coords, int64_t n_points, 
     const PropArgs P = prop_args(coords, n_points, warp, box_size, embeddings, offsets, num_levels, S, H, gridtype,
                                  align_corners, interp, w1, b1, w2, b2, density_bias);
     int64_t nb;
-    st = prop_blocks(n_points, PF_BWD_THREADS, 3, &nb);
-    if (st) return st;
     hipStream_t s = (hipStream_t)stream;
 #define LAUNCH_PB(CC, FM, FX)                                                                                    \
+    st = prop_blocks(n_points, pf_bwd_threads(FM), 768 / pf_bwd_threads(FM), &nb);                              \
+    if (st) return st;                                                                                          \
     if (dtype == 0)                                                                                              \
-        hipLaunchKernelGGL((prop_bwd_kernel<float, CC, FM, FX>), dim3((unsigned)nb), dim3(PF_BWD_THREADS), 0, s, \
+        hipLaunchKernelGGL((prop_bwd_kernel<float, CC, FM, FX>), dim3((unsigned)nb), dim3(pf_bwd_threads(FM)), 0, s, \
                            P, grad_density, features, grad_features, grid_inputs, grad_w1, grad_b1, grad_w2,     \
                            grad_b2);                                                                             \
     else                                                                                                         \
-        hipLaunchKernelGGL((prop_bwd_kernel<__half, CC, FM, FX>), dim3((unsigned)nb), dim3(PF_BWD_THREADS), 0,   \
+        hipLaunchKernelGGL((prop_bwd_kernel<__half, CC, FM, FX>), dim3((unsigned)nb), dim3(pf_bwd_threads(FM)), 0,   \
                            s, P, grad_density, features, grad_features, grid_inputs, grad_w1, grad_b1, grad_w2,  \
                            grad_b2);
     const bool small = num_levels * level_dim <= 16;

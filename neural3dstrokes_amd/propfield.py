@@ -47,10 +47,14 @@ class _prop_field_fn(Function):
         # the encoder's outputs (F floats per point) and inputs, kept so the adjoint gathers nothing
         feats = torch.empty(N, L * C, dtype=torch.float32, device=dev) if keep else None
         x01 = torch.empty(N, 3, dtype=torch.float32, device=dev) if keep else None
-        _lib.check(_lib.lib().n3ds_prop_field_forward(
+        rows, flag = embeddings.shape[0], _grid._dtype_flag(embeddings)
+        nws = int(_lib.lib().n3ds_prop_field_workspace_bytes(N, L, C, rows, flag))
+        ws = torch.empty(nws, dtype=torch.uint8, device=dev) if nws > 0 else None
+        _lib.check(_lib.lib().n3ds_prop_field_forward_ws(
             _lib.ptr(coords), N, warp, float(box), _lib.ptr(embeddings), _lib.ptr(offsets), L, C, S, H, gridtype,
-            align, interp, _grid._dtype_flag(embeddings), _lib.ptr(w1), _lib.ptr(b1), _lib.ptr(w2), _lib.ptr(b2),
-            float(dbias), _lib.ptr(density), _lib.ptr(coord), _lib.ptr(feats), _lib.ptr(x01), _lib.stream()))
+            align, interp, flag, _lib.ptr(w1), _lib.ptr(b1), _lib.ptr(w2), _lib.ptr(b2), float(dbias),
+            _lib.ptr(density), _lib.ptr(coord), _lib.ptr(feats), _lib.ptr(x01), rows, _lib.ptr(ws), max(nws, 0),
+            _lib.stream()))
         empty = torch.empty(0, device=dev)
         ctx.save_for_backward(coords, embeddings, w1, b1, w2, b2, feats if keep else empty, x01 if keep else empty)
         ctx.cfg = cfg
