@@ -37,14 +37,9 @@ __device__ __forceinline__ float sf_wave_max(float v) {
 }
 
 // the inverse CDF at u (sorted_interp(u, cw0, t) for non-decreasing cw0, sorted t)
-__device__ __forceinline__ float sf_center(const float* cw, const float* te, int m, float u) {
-    int lo = 0, hi = m + 1;  // first index with cw[idx] > u, in [1, m] after the clamp
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (cw[mid] <= u) lo = mid + 1;
-        else hi = mid;
-    }
-    const int k = min(max(lo, 1), m);
+// first: the first index with cw[idx] > u, in [1, m] after the clamp
+__device__ __forceinline__ float sf_center(const float* cw, const float* te, int m, float u, int first) {
+    const int k = min(max(first, 1), m);
     const float x0 = cw[k - 1], x1 = cw[k], f0 = te[k - 1], f1 = te[k];
     float off = (u - x0) / (x1 - x0);
     if (off != off) off = 0.f;  // nan_to_num(., 0)
@@ -52,6 +47,23 @@ __device__ __forceinline__ float sf_center(const float* cw, const float* te, int
     return __fadd_rn(f0, __fmul_rn(off, __fsub_rn(f1, f0)));
 }
 
+// 64 entries of cw0 = [0, min(cumsum(w[:-1]), 1), 1]: lane's weight v of bin j after the
+// running sum carry; returns the sum so far
+__device__ __forceinline__ float sf_cdf(float* cw, int j, int m, float v, float carry, int lane) {
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const float o = __shfl_up(v, off, 64);
+        if (lane >= off) v += o;
+    }
+    v += carry;
+    if (j < m - 1) cw[j + 1] = fminf(v, 1.f);
+    return __shfl(v, 63, 64);
+}
+
+// NB > 0: at most 64 NB bins, their logits and exponentials in registers (0: any number, read
+// and exponentiated again for each use): 67 instead of 75 us at 65536 rays, 192 bins and 128
+// samples, with the two searches of a lane side by side.
+template <int NB>
 __global__ __launch_bounds__(256) void sample_intervals_kernel(float* __restrict__ t_out,
                                                                const float* __restrict__ t,
                                                                const float* __restrict__ logits,
@@ -68,25 +80,38 @@ __global__ __launch_bounds__(256) void sample_intervals_kernel(float* __restrict
         const float* tr = t + r * (m + 1);
         const float* lr = logits + r * m;
         // softmax over the m bins
-        float mx = -INFINITY;
-        for (int j = lane; j < m; j += 64) mx = fmaxf(mx, lr[j]);
-        mx = sf_wave_max(mx);
-        float se = 0.f;
-        for (int j = lane; j < m; j += 64) se += expf(lr[j] - mx);
-        se = wave_sum(se);
-        // cw0 = [0, min(cumsum(w[:-1]), 1), 1]
         float carry = 0.f;
-        for (int j0 = 0; j0 < m - 1; j0 += 64) {
-            const int j = j0 + lane;
-            float v = j < m - 1 ? expf(lr[j] - mx) / se : 0.f;
+        if constexpr (NB > 0) {
+            float v[NB], mx = -INFINITY, se = 0.f;
 #pragma unroll
-            for (int off = 1; off < 64; off <<= 1) {
-                const float o = __shfl_up(v, off, 64);
-                if (lane >= off) v += o;
+            for (int s = 0; s < NB; s++) {
+                v[s] = lane + 64 * s < m ? lr[lane + 64 * s] : -INFINITY;
+                mx = fmaxf(mx, v[s]);
             }
-            v += carry;
-            if (j < m - 1) cw[j + 1] = fminf(v, 1.f);
-            carry = __shfl(v, 63, 64);
+            mx = sf_wave_max(mx);
+#pragma unroll
+            for (int s = 0; s < NB; s++)
+                if (lane + 64 * s < m) {
+                    v[s] = expf(v[s] - mx);
+                    se += v[s];
+                }
+            se = wave_sum(se);
+#pragma unroll
+            for (int s = 0; s < NB; s++) {
+                const int j = lane + 64 * s;
+                carry = sf_cdf(cw, j, m, j < m - 1 ? v[s] / se : 0.f, carry, lane);
+            }
+        } else {
+            float mx = -INFINITY;
+            for (int j = lane; j < m; j += 64) mx = fmaxf(mx, lr[j]);
+            mx = sf_wave_max(mx);
+            float se = 0.f;
+            for (int j = lane; j < m; j += 64) se += expf(lr[j] - mx);
+            se = wave_sum(se);
+            for (int j0 = 0; j0 < m - 1; j0 += 64) {
+                const int j = j0 + lane;
+                carry = sf_cdf(cw, j, m, j < m - 1 ? expf(lr[j] - mx) / se : 0.f, carry, lane);
+            }
         }
         if (lane == 0) {
             cw[0] = 0.f;
@@ -96,10 +121,25 @@ __global__ __launch_bounds__(256) void sample_intervals_kernel(float* __restrict
         sf_wave_sync();
         float* outr = t_out + r * (n + 1);
         const float* jr = jitter ? jitter + r * jitter_width : nullptr;
-        for (int i = lane; i < n; i += 64) {
-            float u = u_base[i];
-            if (jr) u = __fadd_rn(u, __fmul_rn(jr[jitter_width == 1 ? 0 : i], max_jitter));
-            cs[i] = sf_center(cw, te, m, u);
+        for (int i = lane; i < n; i += 128) {  // two searches side by side
+            const int i1 = i + 64 < n ? i + 64 : i;
+            float u0 = u_base[i], u1 = u_base[i1];
+            if (jr) {
+                u0 = __fadd_rn(u0, __fmul_rn(jr[jitter_width == 1 ? 0 : i], max_jitter));
+                u1 = __fadd_rn(u1, __fmul_rn(jr[jitter_width == 1 ? 0 : i1], max_jitter));
+            }
+            int lo0 = 0, hi0 = m + 1, lo1 = 0, hi1 = m + 1;  // first index with cw[idx] > u
+            for (int left = m + 1; left > 0; left >>= 1) {
+                const int mid0 = (lo0 + hi0) >> 1, mid1 = (lo1 + hi1) >> 1;
+                const bool le0 = cw[min(mid0, m)] <= u0, le1 = cw[min(mid1, m)] <= u1;
+                const bool go0 = lo0 < hi0, go1 = lo1 < hi1;
+                if (go0 && le0) lo0 = mid0 + 1;
+                if (go0 && !le0) hi0 = mid0;
+                if (go1 && le1) lo1 = mid1 + 1;
+                if (go1 && !le1) hi1 = mid1;
+            }
+            cs[i] = sf_center(cw, te, m, u0, lo0);
+            if (i + 64 < n) cs[i1] = sf_center(cw, te, m, u1, lo1);
         }
         sf_wave_sync();
         for (int o = lane; o <= n; o += 64) {
@@ -368,9 +408,14 @@ N3DS_EXPORT int n3ds_sample_intervals(float* t_out, const float* t, const float*
     const int waves = per_wave <= SF_MAX_FLOATS / 4 ? 4 : 1;
     const size_t lds = (size_t)waves * per_wave * sizeof(float);
     const int64_t blocks = std::min<int64_t>((n_rays + waves - 1) / waves, 256 * 32);
-    hipLaunchKernelGGL(sample_intervals_kernel, dim3((unsigned)blocks), dim3(64 * waves), lds, (hipStream_t)stream,
-                       t_out, t, w_logits, u_base, jitter, jitter_width, max_jitter, n_rays, n_bins, n_samples,
-                       minval, maxval, waves);
+    typedef void (*Kernel)(float*, const float*, const float*, const float*, const float*, int, float, int64_t, int,
+                           int, float, float, int);
+    static const Kernel kernels[5] = {sample_intervals_kernel<0>, sample_intervals_kernel<1>,
+                                      sample_intervals_kernel<2>, sample_intervals_kernel<3>,
+                                      sample_intervals_kernel<4>};
+    hipLaunchKernelGGL(kernels[n_bins <= 256 ? (n_bins + 63) / 64 : 0], dim3((unsigned)blocks), dim3(64 * waves), lds,
+                       (hipStream_t)stream, t_out, t, w_logits, u_base, jitter, jitter_width, max_jitter, n_rays,
+                       n_bins, n_samples, minval, maxval, waves);
     N3DS_LAUNCH_CHECK();
     return N3DS_OK;
 }
