@@ -17,8 +17,13 @@ from . import _lib
 
 def resample_logits(sdist, weights, resample_padding=0.0):
     """models.py:168-171: log(w + padding) on bins of positive width, -inf elsewhere."""
-    return torch.where(sdist[..., 1:] > sdist[..., :-1], torch.log(weights + resample_padding),
-                       torch.full_like(sdist[..., :-1], -torch.inf))
+    # three elementwise passes instead of five: log of -0 and of 0 are the same, and -inf needs
+    # no tensor of its own where it does not decide the result's type
+    padded = weights if isinstance(resample_padding, (int, float)) and resample_padding == 0 else \
+        weights + resample_padding
+    logits = torch.log(padded)
+    empty = -torch.inf if logits.dtype == sdist.dtype else torch.full_like(sdist[..., :-1], -torch.inf)
+    return torch.where(sdist[..., 1:] > sdist[..., :-1], logits, empty)
 
 
 def sample_intervals(rand, t, w_logits, num_samples, single_jitter=False, domain=(-torch.inf, torch.inf)):
