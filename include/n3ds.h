@@ -147,20 +147,6 @@ int n3ds_prop_field_forward(const float* coords, int64_t n_points, int warp, flo
                             const float* w2, const float* b2, float density_bias, float* density_out,
                             float* coord_out, float* features_out, float* grid_inputs_out, void* stream);
 
-/* The same with device scratch: for many points of tables larger than an L2 the
- * grid features are gathered level by level over all points first.
- * n_rows: rows of the whole table.  workspace: at least
- * n3ds_prop_field_workspace_bytes() (0 where the one kernel is the faster way);
- * with NULL or fewer bytes it runs as n3ds_prop_field_forward. */
-int64_t n3ds_prop_field_workspace_bytes(int64_t n_points, int num_levels, int level_dim, int64_t n_rows, int dtype);
-int n3ds_prop_field_forward_ws(const float* coords, int64_t n_points, int warp, float box_size,
-                               const void* embeddings, const int32_t* offsets, int num_levels, int level_dim,
-                               float S, int H, int gridtype, int align_corners, int interp, int dtype,
-                               const float* w1, const float* b1, const float* w2, const float* b2,
-                               float density_bias, float* density_out, float* coord_out, float* features_out,
-                               float* grid_inputs_out, int64_t n_rows, void* workspace, int64_t workspace_bytes,
-                               void* stream);
-
 /* Adjoint of n3ds_prop_field_forward for upstream grad_density [N]: reads the
  * kept features [N, F] (or, when NULL, gathers them again from the table and
  * writes grid_inputs [N,3]), recomputes the hidden units per point (the [N, 64]

@@ -37,9 +37,6 @@ SIGNATURES = {
     'n3ds_grid_grad_tv': (_I32, [_P, _P, _P, _P, _F, _I64, _I32, _I32, _I32, _F, _I32, _I32, _I32, _I32, _P]),
     'n3ds_prop_field_forward': (_I32, [_P, _I64, _I32, _F, _P, _P, _I32, _I32, _F, _I32, _I32, _I32, _I32, _I32, _P,
                                        _P, _P, _P, _F, _P, _P, _P, _P, _P]),
-    'n3ds_prop_field_workspace_bytes': (_I64, [_I64, _I32, _I32, _I64, _I32]),
-    'n3ds_prop_field_forward_ws': (_I32, [_P, _I64, _I32, _F, _P, _P, _I32, _I32, _F, _I32, _I32, _I32, _I32, _I32, _P,
-                                          _P, _P, _P, _F, _P, _P, _P, _P, _I64, _P, _I64, _P]),
     'n3ds_prop_field_backward': (_I32, [_P, _I64, _I32, _F, _P, _P, _I32, _I32, _F, _I32, _I32, _I32, _I32, _I32, _P,
                                         _P, _P, _P, _F, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
     'n3ds_grad_sqnorm_accumulate': (_I32, [_P, _I64, _P, _P]),
@@ -77,6 +74,14 @@ SIGNATURES = {
     'n3ds_texture_backward': (_I32, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _D, _I32, _P]),
 }
 
+# entry points of this package only, not of the C interface (n3ds.h): n3ds_prop_field_forward with
+# device scratch, and the scratch it wants (0 where one kernel is the faster way)
+INTERNAL = {
+    'n3ds_prop_field_workspace_bytes': (_I64, [_I64, _I32, _I32, _I64, _I32]),
+    'n3ds_prop_field_forward_ws': (_I32, [_P, _I64, _I32, _F, _P, _P, _I32, _I32, _F, _I32, _I32, _I32, _I32, _I32, _P,
+                                          _P, _P, _P, _F, _P, _P, _P, _P, _I64, _P, _I64, _P]),
+}
+
 _lib = None
 
 
@@ -87,7 +92,7 @@ def lib():
         if not os.path.exists(LIB_PATH):
             raise RuntimeError(f'{LIB_PATH} is not built; run `python -m neural3dstrokes_amd.build`')
         handle = ctypes.CDLL(LIB_PATH)
-        for name, (res, args) in SIGNATURES.items():
+        for name, (res, args) in {**SIGNATURES, **INTERNAL}.items():
             fn = getattr(handle, name)
             fn.restype = res
             fn.argtypes = args

@@ -1901,6 +1901,8 @@ N3DS_EXPORT int64_t n3ds_prop_field_workspace_bytes(int64_t n_points, int num_le
     return std::min(n_points, PF_STAGE_CHUNK) * num_levels * level_dim * 4;
 }
 
+// n3ds_prop_field_forward with device scratch of n3ds_prop_field_workspace_bytes (n_rows: rows of
+// the whole table); with NULL or fewer bytes, or where that is 0, one kernel as without it.
 N3DS_EXPORT int n3ds_prop_field_forward_ws(const float* coords, int64_t n_points, int warp, float box_size,
                                            const void* embeddings, const int32_t* offsets, int num_levels,
                                            int level_dim, float S, int H, int gridtype, int align_corners, int interp,
