@@ -83,7 +83,7 @@ __device__ __forceinline__ float compose_front(const float* __restrict__ arow, c
         }
     }
 #pragma unroll
-    for (int c = 0; c <= D; c++) out[c] = wave_sum(sum[c]);
+    for (int c = 0; c <= D; c++) out[c] = wave_sum_halves(sum[c]);  // (wave_sum: adjoint 2 % slower)
     return T;
 }
 

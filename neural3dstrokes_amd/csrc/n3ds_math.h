@@ -47,10 +47,50 @@ __device__ __forceinline__ int lane_i(int v, int j) { return __builtin_amdgcn_re
 __device__ __forceinline__ float lane_f(float v, int j) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j));
 }
-__device__ __forceinline__ float wave_sum(float v) {
+// Scans and reductions over the wavefront's lanes, all of them active, by data-parallel
+// moves inside the vector registers: rows of 16 lanes are shifted by 1, 2, 4 and 8, then a
+// row's last lane is carried to the next row and lane 31 to the upper half.  Six dependent
+// vector instructions; the same steps as shuffles are six round trips through the LDS with
+// three more instructions each.  With them the forward takes 310 instead of 333 us (500 strokes,
+// 65536 rays x 128 samples) and 5242 instead of 5515 (1000, 640000 x 192), its extras 674 instead
+// of 811, the culling pass 174 instead of 178.  Sums round in another order than by halves.
+// The lane a step takes from, or old where there is none.
+template <int STEP>
+__device__ __forceinline__ int lane_before(int old, int v) {
+    constexpr int ctrl[6] = {0x111, 0x112, 0x114, 0x118, 0x142, 0x143};  // row_shr 1, 2, 4, 8; row_bcast 15, 31
+    constexpr int rows[6] = {0xf, 0xf, 0xf, 0xf, 0xa, 0xc};
+    return __builtin_amdgcn_update_dpp(old, v, ctrl[STEP], rows[STEP], 0xf, false);
+}
+template <int STEP>
+__device__ __forceinline__ float lane_before(float old, float v) {
+    return __int_as_float(lane_before<STEP>(__float_as_int(old), __float_as_int(v)));
+}
+// inclusive scan; id: what op leaves as it is
+template <typename T, typename Op>
+__device__ __forceinline__ T wave_scan(T v, T id, Op op) {
+    v = op(lane_before<0>(id, v), v);
+    v = op(lane_before<1>(id, v), v);
+    v = op(lane_before<2>(id, v), v);
+    v = op(lane_before<3>(id, v), v);
+    v = op(lane_before<4>(id, v), v);
+    v = op(lane_before<5>(id, v), v);
+    return v;
+}
+__device__ __forceinline__ float wave_scan_sum(float v) {
+    return wave_scan(v, 0.f, [](float a, float b) { return a + b; });
+}
+__device__ __forceinline__ float wave_sum(float v) { return lane_f(wave_scan_sum(v), 63); }
+// the sum by halves of the wavefront, through the LDS: other roundings than wave_sum's
+__device__ __forceinline__ float wave_sum_halves(float v) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
     return v;
+}
+__device__ __forceinline__ float wave_max(float v) {
+    return lane_f(wave_scan(v, -INFINITY, [](float a, float b) { return fmaxf(a, b); }), 63);
+}
+__device__ __forceinline__ float wave_min(float v) {
+    return lane_f(wave_scan(v, INFINITY, [](float a, float b) { return fminf(a, b); }), 63);
 }
 
 }  // namespace n3ds

@@ -566,13 +566,8 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__device__ __forceinline__ int wave_incl_scan(int v, int lane) {
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        int u = __shfl_up(v, off, 64);
-        if (lane >= off) v += u;
-    }
-    return v;
+__device__ __forceinline__ int wave_incl_scan(int v) {
+    return wave_scan(v, 0, [](int a, int b) { return a + b; });
 }
 
 // Hits are gathered over consecutive 64-stroke chunks (in compositing order)
@@ -665,7 +660,7 @@ __device__ __forceinline__ int class_sort_hits(const WaveMem& w, int hc, int hcl
     for (int x = 0; x < NCLASS; x++) {
         const bool in = hcls == x;
         const unsigned long long m = __ballot(in);
-        const int incl = wave_incl_scan(in ? cnt : 0, lane);
+        const int incl = wave_incl_scan(in ? cnt : 0);
         if (in) {
             rank = before_hits + __popcll(m & ((1ull << lane) - 1ull));
             xo = before_pairs + incl - cnt;
@@ -860,7 +855,7 @@ __device__ __forceinline__ int append_hits(const RenderArgs& A, const RayConst& 
     const bool hit = cull_chunk<NS>(A, rc, w, sorted, base0, lane, k, i0, cnt, cls, pmask);
     const bool curve = cls < 2;
     const unsigned long long mask = __ballot(hit);
-    const int incl = wave_incl_scan(hit ? cnt : 0, lane);
+    const int incl = wave_incl_scan(hit ? cnt : 0);
     if (hit) {
         const int rank = nh + __popcll(mask & ((1ull << lane) - 1ull));
         w.ck[rank] = k;
@@ -944,7 +939,7 @@ __device__ __forceinline__ int refine_pending(const RenderArgs& A, const RayCons
         }
         const bool keep = c < nh && cnt > 0;
         const unsigned long long km = __ballot(keep);
-        const int incl = wave_incl_scan(keep ? cnt : 0, lane);
+        const int incl = wave_incl_scan(keep ? cnt : 0);
         wave_sync();  // every lane has read its entry before any is overwritten (new index <= old)
         if (keep) {
             const int r = out + __popcll(km & ((1ull << lane) - 1ull));
@@ -1148,7 +1143,7 @@ __global__ __launch_bounds__(64 * CWAVES) void render_cull_kernel(RenderArgs A0,
                 const int st = ist[j * 64 + lane];
                 pm = (st & 1) ? ((unsigned)st >> 16) : 0u;
                 np = __popc(pm);
-                incl = wave_incl_scan(np, lane);
+                incl = wave_incl_scan(np);
                 tot = lane_i(incl, 63);
             }
             int done = 0;
@@ -1217,7 +1212,7 @@ __global__ __launch_bounds__(64 * CWAVES) void render_cull_kernel(RenderArgs A0,
                 }
             }
             const unsigned long long mask = __ballot(hit);
-            const int incl = wave_incl_scan(hit ? cnt : 0, lane);
+            const int incl = wave_incl_scan(hit ? cnt : 0);
             if (hit) slots[slot * 64 + __popcll(mask & ((1ull << lane) - 1ull))] = pack_hit(lane, i0, cnt, cls);
             const int tot = lane_i(incl, 63);
             if (lane == 0) counts[slot] = __popcll(mask) | (tot << 8);
@@ -1616,7 +1611,7 @@ __global__ __launch_bounds__(64 * CWAVES) void render_cull_grid_kernel(RenderArg
         lane >= nch ? 0ull
                     : (sorted ? rmask[ray * nch + lane] : (nvalid >= 64 ? ~0ull : ((1ull << nvalid) - 1ull)));
     const int pc = __popcll(mj);
-    const int pincl = wave_incl_scan(pc, lane);
+    const int pincl = wave_incl_scan(pc);
     if (lane < nch) {
         cfirst[lane] = pincl - pc;
         chits[lane] = 0;
@@ -1706,7 +1701,7 @@ __global__ __launch_bounds__(64 * CWAVES) void render_cull_grid_kernel(RenderArg
                 const int st = q < nc ? ist[q] : 0;
                 pm = (st & 1) ? ((unsigned)st >> 16) : 0u;
                 npc = __popc(pm);
-                incl = wave_incl_scan(npc, lane);
+                incl = wave_incl_scan(npc);
                 tot = lane_i(incl, 63);
             }
             int done = 0;
@@ -1848,7 +1843,7 @@ __device__ __forceinline__ void render_fwd_body(const RenderArgs& A0, float* __r
             const int64_t slot0 = ray * A.nch_stride;
             cword = lane < A.nch ? A.ccounts[slot0 + lane] : 0;
             const int ncl = cword & 127;
-            const int hincl = wave_incl_scan(ncl, lane);
+            const int hincl = wave_incl_scan(ncl);
             const int H = lane_i(hincl, 63);
             if (H <= HMAX) {
                 w.xo[lane] = hincl - ncl;
@@ -1864,7 +1859,7 @@ __device__ __forceinline__ void render_fwd_body(const RenderArgs& A0, float* __r
                         hw = A.cslots[(slot0 + c) * 64 + (hi - w.xo[c])];
                         cnt = (hw >> 15) & 511;
                     }
-                    const int incl = wave_incl_scan(cnt, lane);
+                    const int incl = wave_incl_scan(cnt);
                     if (hi < H) {
                         w.ck[hi] = A.S - 1 - (c * 64 + (hw & 63));
                         w.ci0[hi] = (hw >> 6) & 511;
@@ -1895,7 +1890,7 @@ __device__ __forceinline__ void render_fwd_body(const RenderArgs& A0, float* __r
             if (nc) {
                 const int hw = lane < nc ? A.cslots[slot * 64 + lane] : 0;
                 const int cnt = lane < nc ? (hw >> 15) & 511 : 0;
-                const int incl = wave_incl_scan(cnt, lane);
+                const int incl = wave_incl_scan(cnt);
                 if (lane < nc) {
                     w.ck[nh + lane] = A.S - 1 - (ch * 64 + (hw & 63));
                     w.ci0[nh + lane] = (hw >> 6) & 511;
@@ -2064,12 +2059,7 @@ __device__ __forceinline__ void render_fwd_body(const RenderArgs& A0, float* __r
     float acc = 0.f, r0 = 0.f, r1 = 0.f, r2 = 0.f, dsum = 0.f;
 #pragma unroll
     for (int s = 0; s < NS; s++) {
-        float v = sd[s];
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const float u = __shfl_up(v, off, 64);
-            if (lane >= off) v += u;
-        }
+        const float v = wave_scan_sum(sd[s]);
         const float excl = carry + v - sd[s];
         const float trans = expf(-excl);
         const float al = (A.opaque && lane + 64 * s == A.n - 1) ? 1.f : 1.f - expf(-sd[s]);
@@ -2142,7 +2132,7 @@ __global__ __launch_bounds__(64 * XWAVES) void render_extras_kernel(const float*
         const bool valid = i < n;
         const float ta = valid ? td[i] : 0.f, tb = valid ? td[i + 1] : 0.f;
         const float sd = valid ? dens[i] * ((tb - ta) * dn) : 0.f;
-        float v = sd;
+        float v = sd;  // in the order of these steps: percentiles turn on the last bits of the sums
 #pragma unroll
         for (int off = 1; off < 64; off <<= 1) {
             const float u = __shfl_up(v, off, 64);
@@ -2180,13 +2170,10 @@ __global__ __launch_bounds__(64 * XWAVES) void render_extras_kernel(const float*
     lsum = wave_sum(lsum);
 #pragma unroll
     for (int q = 0; q < 3; q++) {
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            x0[q] = fmaxf(x0[q], __shfl_xor(x0[q], off, 64));
-            f0[q] = fmaxf(f0[q], __shfl_xor(f0[q], off, 64));
-            x1[q] = fminf(x1[q], __shfl_xor(x1[q], off, 64));
-            f1[q] = fminf(f1[q], __shfl_xor(f1[q], off, 64));
-        }
+        x0[q] = wave_max(x0[q]);
+        f0[q] = wave_max(f0[q]);
+        x1[q] = wave_min(x1[q]);
+        f1[q] = wave_min(f1[q]);
     }
     if (lane == 0) {
         float dm = expf(lsum / fmaxf(acc, 1.1920929e-07f));
@@ -2434,7 +2421,7 @@ static_assert(SP_PAGE >= PBUF && SP_PAGE % 64 == 0, "a window fits one new page"
 
 // One block: the group counts of the pages handed out replaced by their exclusive prefix,
 // the total behind the last; also clears z[0..nz).  Tiles of 4096 counts, four per thread:
-// wavefront scans by shuffles, the 16 wavefront totals through LDS.
+// wavefront scans in registers, the 16 wavefront totals through LDS.
 constexpr int SCAN_THREADS = 1024;
 __global__ __launch_bounds__(SCAN_THREADS) void page_scan_kernel(int* __restrict__ c, const int* __restrict__ next,
                                                                  int first, int pages, float* __restrict__ z,
@@ -2452,7 +2439,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void page_scan_kernel(int* __restrict
             v[q] = i0 + q < n ? c[i0 + q] : 0;
             sum += v[q];
         }
-        const int incl = wave_incl_scan(sum, lane);
+        const int incl = wave_incl_scan(sum);
         if (lane == 63) wtot[wave] = incl;
         __syncthreads();
         int before = 0, total = 0;
@@ -2648,12 +2635,7 @@ __global__ __launch_bounds__(64 * BWAVES) void render_bwd_kernel(RenderArgs A0, 
         float carry = 0.f, acc = 0.f, dsum = 0.f;
 #pragma unroll
         for (int s = 0; s < NS; s++) {
-            float v = sdl[s];
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) {
-                const float u = __shfl_up(v, off, 64);
-                if (lane >= off) v += u;
-            }
+            const float v = wave_scan_sum(sdl[s]);
             const float excl = carry + v - sdl[s];
             trv[s] = expf(-excl);
             const float al = (A.opaque && lane + 64 * s == A.n - 1) ? 1.f : 1.f - expf(-sdl[s]);

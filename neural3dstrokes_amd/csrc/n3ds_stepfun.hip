@@ -30,12 +30,6 @@ __device__ __forceinline__ void sf_wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__device__ __forceinline__ float sf_wave_max(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-    return v;
-}
-
 // the inverse CDF at u (sorted_interp(u, cw0, t) for non-decreasing cw0, sorted t)
 // first: the first index with cw[idx] > u, in [1, m] after the clamp
 __device__ __forceinline__ float sf_center(const float* cw, const float* te, int m, float u, int first) {
@@ -88,14 +82,14 @@ __global__ __launch_bounds__(256) void sample_intervals_kernel(float* __restrict
                 v[s] = lane + 64 * s < m ? lr[lane + 64 * s] : -INFINITY;
                 mx = fmaxf(mx, v[s]);
             }
-            mx = sf_wave_max(mx);
+            mx = wave_max(mx);
 #pragma unroll
             for (int s = 0; s < NB; s++)
                 if (lane + 64 * s < m) {
                     v[s] = expf(v[s] - mx);
                     se += v[s];
                 }
-            se = wave_sum(se);
+            se = wave_sum_halves(se);  // (a sample's bin may turn on its last bit)
 #pragma unroll
             for (int s = 0; s < NB; s++) {
                 const int j = lane + 64 * s;
@@ -104,10 +98,10 @@ __global__ __launch_bounds__(256) void sample_intervals_kernel(float* __restrict
         } else {
             float mx = -INFINITY;
             for (int j = lane; j < m; j += 64) mx = fmaxf(mx, lr[j]);
-            mx = sf_wave_max(mx);
+            mx = wave_max(mx);
             float se = 0.f;
             for (int j = lane; j < m; j += 64) se += expf(lr[j] - mx);
-            se = wave_sum(se);
+            se = wave_sum_halves(se);
             for (int j0 = 0; j0 < m - 1; j0 += 64) {
                 const int j = j0 + lane;
                 carry = sf_cdf(cw, j, m, j < m - 1 ? expf(lr[j] - mx) / se : 0.f, carry, lane);
@@ -240,7 +234,7 @@ __device__ __forceinline__ void dilate_ray(float* __restrict__ t_out, float* __r
         wsum += wd;
     }
     if (renormalize) {
-        wsum = fmaxf(wave_sum(wsum), eps);
+        wsum = fmaxf(wave_sum_halves(wsum), eps);
         for (int i = lane; i < ne - 1; i += 64) wout[i] = wout[i] / wsum;
     }
 }
@@ -379,7 +373,7 @@ __global__ __launch_bounds__(256) void max_dilate_small_kernel(float* __restrict
             }
         }
         if (ne > 192 && lane == 0) tout[ne - 1] = es[ne - 1];
-        if (renormalize) wsum = fmaxf(wave_sum(wsum), eps);
+        if (renormalize) wsum = fmaxf(wave_sum_halves(wsum), eps);
 #pragma unroll
         for (int s = 0; s < 3; s++) {
             const int i = lane + 64 * s;
