@@ -75,11 +75,14 @@ SIGNATURES = {
 }
 
 # entry points of this package only, not of the C interface (n3ds.h): n3ds_prop_field_forward with
-# device scratch, and the scratch it wants (0 where one kernel is the faster way)
+# device scratch, and the scratch it wants (0 where one kernel is the faster way);
+# n3ds_prop_field_backward with its weight gradients summed in doubles
 INTERNAL = {
     'n3ds_prop_field_workspace_bytes': (_I64, [_I64, _I32, _I32, _I64, _I32]),
     'n3ds_prop_field_forward_ws': (_I32, [_P, _I64, _I32, _F, _P, _P, _I32, _I32, _F, _I32, _I32, _I32, _I32, _I32, _P,
                                           _P, _P, _P, _F, _P, _P, _P, _P, _I64, _P, _I64, _P]),
+    'n3ds_prop_field_backward_sums': (_I32, [_P, _I64, _I32, _F, _P, _P, _I32, _I32, _F, _I32, _I32, _I32, _I32, _I32,
+                                             _P, _P, _P, _P, _F, _P, _P, _P, _P, _P, _P]),
 }
 
 _lib = None

@@ -1506,7 +1506,8 @@ __global__ __launch_bounds__(pf_bwd_threads(FM)) void prop_bwd_kernel(PropArgs P
                                                                   const float* __restrict__ feat_in,
                                                                   float* __restrict__ gfeat, float* __restrict__ x01_out,
                                                                   float* __restrict__ gW1, float* __restrict__ gb1,
-                                                                  float* __restrict__ gW2, float* __restrict__ gb2) {
+                                                                  float* __restrict__ gW2, float* __restrict__ gb2,
+                                                                  double* __restrict__ gsum) {
     constexpr int NT = pf_bwd_threads(FM), NW = NT / 64, KS = (FM + 3) / 4, FT = (FM + 15) / 16, HT = PF_HID / 16;
     constexpr int FP = 16 * FT + 1;  // row of a point's features in LDS
     __shared__ float sf[NW][64][FP];  // a wavefront's 64 points: features, then their gradients
@@ -1535,7 +1536,8 @@ __global__ __launch_bounds__(pf_bwd_threads(FM)) void prop_bwd_kernel(PropArgs P
     }
     const float b2 = P.b2[0];
     f4 aw1[FT][HT];
-    float ab1[HT], aw2[HT], ab2 = 0.f;
+    float ab1[HT], aw2[HT];
+    double ab2 = 0.0;  // 16 lanes take all of the wavefront's points: in float32 less exact than a lane per point
 #pragma unroll
     for (int t = 0; t < HT; t++) {
         ab1[t] = aw2[t] = 0.f;
@@ -1596,7 +1598,7 @@ __global__ __launch_bounds__(pf_bwd_threads(FM)) void prop_bwd_kernel(PropArgs P
             raw += __shfl_xor(raw, 16, 64);
             raw += __shfl_xor(raw, 32, 64);
             const float g = __shfl(gown, 16 * s + lc, 64) * dsoftplus20(raw + b2 + P.dbias);
-            if (lr == 0) ab2 += g;
+            if (lr == 0) ab2 += (double)g;
             f4 df[FT];
 #pragma unroll
             for (int q = 0; q < FT; q++) df[q] = (f4){0.f, 0.f, 0.f, 0.f};
@@ -1652,8 +1654,13 @@ __global__ __launch_bounds__(pf_bwd_threads(FM)) void prop_bwd_kernel(PropArgs P
         atomicAdd(&sum[PF_HID * FM + j], (double)ab1[t]);
         atomicAdd(&sum[PF_HID * (FM + 1) + j], (double)aw2[t]);
     }
-    if (lr == 0) atomicAdd(&sum[PF_HID * (FM + 2)], (double)ab2);
+    if (lr == 0) atomicAdd(&sum[PF_HID * (FM + 2)], ab2);
     __syncthreads();
+    if (gsum) {  // [W1 | b1 | W2 | b2] in doubles: the order of the blocks leaves no rounding in them
+        for (int i = threadIdx.x; i < PF_HID * (F + 2) + 1; i += NT)
+            atomicAdd(&gsum[i], i < PF_HID * F ? sum[(i / F) * FM + i % F] : sum[PF_HID * FM + i - PF_HID * F]);
+        return;
+    }
     for (int i = threadIdx.x; i < PF_HID * F; i += NT)
         atomicAdd(&gW1[i], (float)sum[(i / F) * FM + i % F]);
     for (int i = threadIdx.x; i < PF_HID; i += NT) {
@@ -1989,7 +1996,7 @@ N3DS_EXPORT int n3ds_prop_field_forward(const float* coords, int64_t n_points, i
                                       density_out, coord_out, features_out, grid_inputs_out, 0, nullptr, 0, stream);
 }
 
-N3DS_EXPORT int n3ds_prop_field_backward(const float* coords, int64_t n_points, int warp, float box_size,
+static int prop_field_backward(double* gsum, const float* coords, int64_t n_points, int warp, float box_size,
                                          const void* embeddings, const int32_t* offsets, int num_levels,
                                          int level_dim, float S, int H, int gridtype, int align_corners, int interp,
                                          int dtype, const float* w1, const float* b1, const float* w2,
@@ -2010,11 +2017,11 @@ N3DS_EXPORT int n3ds_prop_field_backward(const float* coords, int64_t n_points, 
     if (dtype == 0)                                                                                              \
         hipLaunchKernelGGL((prop_bwd_kernel<float, CC, FM, FX>), dim3((unsigned)nb), dim3(pf_bwd_threads(FM)), 0, s, \
                            P, grad_density, features, grad_features, grid_inputs, grad_w1, grad_b1, grad_w2,     \
-                           grad_b2);                                                                             \
+                           grad_b2, gsum);                                                                             \
     else                                                                                                         \
         hipLaunchKernelGGL((prop_bwd_kernel<__half, CC, FM, FX>), dim3((unsigned)nb), dim3(pf_bwd_threads(FM)), 0,   \
                            s, P, grad_density, features, grad_features, grid_inputs, grad_w1, grad_b1, grad_w2,  \
-                           grad_b2);
+                           grad_b2, gsum);
     const bool small = num_levels * level_dim <= 16;
     if (level_dim == 1 && num_levels == 10) {
         LAUNCH_PB(1, 12, 10)
@@ -2030,4 +2037,32 @@ N3DS_EXPORT int n3ds_prop_field_backward(const float* coords, int64_t n_points, 
 #undef LAUNCH_PB
     N3DS_LAUNCH_CHECK();
     return N3DS_OK;
+}
+
+N3DS_EXPORT int n3ds_prop_field_backward(const float* coords, int64_t n_points, int warp, float box_size,
+                                         const void* embeddings, const int32_t* offsets, int num_levels,
+                                         int level_dim, float S, int H, int gridtype, int align_corners, int interp,
+                                         int dtype, const float* w1, const float* b1, const float* w2,
+                                         const float* b2, float density_bias, const float* grad_density,
+                                         const float* features, float* grad_features, float* grid_inputs,
+                                         float* grad_w1, float* grad_b1, float* grad_w2, float* grad_b2,
+                                         void* stream) {
+    return prop_field_backward(nullptr, coords, n_points, warp, box_size, embeddings, offsets, num_levels,
+                               level_dim, S, H, gridtype, align_corners, interp, dtype, w1, b1, w2, b2,
+                               density_bias, grad_density, features, grad_features, grid_inputs, grad_w1,
+                               grad_b1, grad_w2, grad_b2, stream);
+}
+
+// n3ds_prop_field_backward with the weight gradients added into grad_sums [64 F | 64 | 64 | 1] doubles
+N3DS_EXPORT int n3ds_prop_field_backward_sums(const float* coords, int64_t n_points, int warp, float box_size,
+                                              const void* embeddings, const int32_t* offsets, int num_levels,
+                                              int level_dim, float S, int H, int gridtype, int align_corners, int interp,
+                                              int dtype, const float* w1, const float* b1, const float* w2,
+                                              const float* b2, float density_bias, const float* grad_density,
+                                              const float* features, float* grad_features, float* grid_inputs,
+                                              double* grad_sums, void* stream) {
+    return prop_field_backward(grad_sums, coords, n_points, warp, box_size, embeddings, offsets, num_levels,
+                               level_dim, S, H, gridtype, align_corners, interp, dtype, w1, b1, w2, b2,
+                               density_bias, grad_density, features, grad_features, grid_inputs, nullptr,
+                               nullptr, nullptr, nullptr, stream);
 }

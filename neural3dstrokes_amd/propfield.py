@@ -70,12 +70,15 @@ class _prop_field_fn(Function):
         Fd = L * C
         g_density = torch.zeros(N, device=dev) if g_density is None else g_density.float().contiguous()
         gfeat = torch.empty(N, Fd, dtype=torch.float32, device=dev)
-        gw1, gb1, gw2, gb2 = (torch.zeros_like(t) for t in (w1, b1, w2, b2))
-        _lib.check(_lib.lib().n3ds_prop_field_backward(
+        # weight gradients [w1 | b1 | w2 | b2], summed over the points in doubles
+        sums = torch.zeros(HIDDEN * (Fd + 2) + 1, dtype=torch.float64, device=dev)
+        _lib.check(_lib.lib().n3ds_prop_field_backward_sums(
             _lib.ptr(coords), N, warp, float(box), _lib.ptr(embeddings), _lib.ptr(offsets), L, C, S, H, gridtype,
             align, interp, _grid._dtype_flag(embeddings), _lib.ptr(w1), _lib.ptr(b1), _lib.ptr(w2), _lib.ptr(b2),
-            float(dbias), _lib.ptr(g_density), _lib.ptr(feats), _lib.ptr(gfeat), _lib.ptr(x01), _lib.ptr(gw1),
-            _lib.ptr(gb1), _lib.ptr(gw2), _lib.ptr(gb2), _lib.stream()))
+            float(dbias), _lib.ptr(g_density), _lib.ptr(feats), _lib.ptr(gfeat), _lib.ptr(x01), _lib.ptr(sums),
+            _lib.stream()))
+        gw1, gb1, gw2, gb2 = (g.reshape(t.shape) for g, t in zip(
+            sums.float().split([HIDDEN * Fd, HIDDEN, HIDDEN, 1]), (w1, b1, w2, b2)))
         g_emb = None
         if ctx.needs_input_grad[1]:
             gfeat_t = gfeat.to(embeddings.dtype).contiguous()
