@@ -1153,8 +1153,8 @@ static int gs_launch(const T* grad, const float* inputs, const int* offsets, int
 constexpr int PF_HID = 64;
 constexpr int PF_MAXF = 32;
 constexpr int PF_FWD_THREADS = 256;
-// Adjoint: one block per CU while its registers allow 12 wavefronts (450 instead of 606 us at
-// 4.2 M points and 10 features; a third of the atomic additions at the end), else three.
+// Adjoint: one block per CU while its registers allow 12 wavefronts (512 us at 4.2 M points and
+// 10 features; without the density's products 450, and 606 with three blocks of four; a third of the atomic additions at the end), else three.
 constexpr int pf_bwd_threads(int fm) { return fm <= 12 ? 768 : 256; }
 
 struct PropArgs {
@@ -1489,17 +1489,20 @@ __device__ __forceinline__ f4 mfma16(float a, float b, f4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// Adjoint of the head.  Its three contractions (hidden units from features, feature
-// gradients from hidden gradients, weight gradients over the points) run on the matrix
-// cores in float32, 16 points at a time:
+// Adjoint of the head.  Its contractions (hidden units from features, the density from the
+// hidden units, feature gradients from hidden gradients, weight gradients over the points) run
+// on the matrix cores in float32, 16 points at a time:
 //   H [hidden x point] = W1 F: the operands' lanes hold W1 and the features; a lane then has
-//     4 hidden units of one point per 16 x 16 tile, sums their W2 relu(H) for the density
-//     and turns them into dH in place, which is at once the right operand of
-//   dF [feature x point] = W1^T dH (the k-th step takes the hidden units 4 (l / 16) + k);
-//   H' [point x hidden] = the same product with its operands exchanged: dH' of it is the
+//     4 hidden units of one point per 16 x 16 tile, at once the right operand of
+//   raw = W2 relu(H), the units in their order, as one lane sums them in the forward (summed
+//     by lanes first, the density's last bits differ: where the bias's gradient cancels over
+//     the points, its error against 64 bits grew from below 1e-6 to above); dH in H's place is
+//     the right operand of
+//   dF [feature x point] = W1^T dH (step r takes the units 4 r + l / 16);
+//   H' [point x hidden] = the first product with its operands exchanged: dH' of it is the
 //     right operand of dW1 [feature x hidden] += F^T dH', summed over all of a wavefront's
 //     points in the accumulator registers.
-// 56 matrix instructions per 16 points and 10 features.  The vector version went through
+// 72 matrix instructions per 16 points and 10 features.  The vector version went through
 // LDS for every product (7 LDS reads per point and hidden unit): 1560 us at 4.2 M points.
 template <typename T, int C, int FM, int FX = 0>
 __global__ __launch_bounds__(pf_bwd_threads(FM)) void prop_bwd_kernel(PropArgs P, const float* __restrict__ gdens,
@@ -1516,23 +1519,26 @@ __global__ __launch_bounds__(pf_bwd_threads(FM)) void prop_bwd_kernel(PropArgs P
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform per wavefront
     const int lc = lane & 15, lr = lane >> 4;
     for (int i = threadIdx.x; i < PF_HID * (FM + 2) + 1; i += NT) sum[i] = 0.0;
-    // constant operands: w1[t][k] = W1[16 t + lc][4 k + lr], w1t[q][t][r] = W1[16 t + 4 lr + r][16 q + lc]
+    // A tile's row 4 a + b is hidden unit 16 t + 4 b + a, so that a lane's r-th unit of H is the
+    // k-th of the r-th step of a product over the units in their order: jl is lc's unit.
+    const int jl = 4 * (lc & 3) + (lc >> 2);
+    // constant operands: w1[t][k] = W1[16 t + jl][4 k + lr], w1t[q][t][r] = W1[16 t + 4 r + lr][16 q + lc]
     float w1[HT][KS], w1t[FT][HT][4], b1q[HT], w2q[HT];
     f4 b1p[HT], w2p[HT];
 #pragma unroll
     for (int t = 0; t < HT; t++) {
 #pragma unroll
-        for (int k = 0; k < KS; k++) w1[t][k] = 4 * k + lr < F ? P.W1[(16 * t + lc) * F + 4 * k + lr] : 0.f;
+        for (int k = 0; k < KS; k++) w1[t][k] = 4 * k + lr < F ? P.W1[(16 * t + jl) * F + 4 * k + lr] : 0.f;
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            const int j = 16 * t + 4 * lr + r;
+            const int j = 16 * t + 4 * r + lr;
 #pragma unroll
             for (int q = 0; q < FT; q++) w1t[q][t][r] = 16 * q + lc < F ? P.W1[j * F + 16 * q + lc] : 0.f;
             b1p[t][r] = P.b1[j];
             w2p[t][r] = P.W2[j];
         }
-        b1q[t] = P.b1[16 * t + lc];
-        w2q[t] = P.W2[16 * t + lc];
+        b1q[t] = P.b1[16 * t + jl];
+        w2q[t] = P.W2[16 * t + jl];
     }
     const float b2 = P.b2[0];
     f4 aw1[FT][HT];
@@ -1590,14 +1596,13 @@ __global__ __launch_bounds__(pf_bwd_threads(FM)) void prop_bwd_kernel(PropArgs P
 #pragma unroll
                 for (int k = 0; k < KS; k++) h[t] = mfma16(w1[t][k], f[k], h[t]);
             }
-            float raw = 0.f;
+            // every row of the product is the density's pre-activation, its 64 terms in order
+            f4 raw = (f4){b2, b2, b2, b2};
 #pragma unroll
             for (int t = 0; t < HT; t++)
 #pragma unroll
-                for (int r = 0; r < 4; r++) raw += w2p[t][r] * fmaxf(h[t][r], 0.f);
-            raw += __shfl_xor(raw, 16, 64);
-            raw += __shfl_xor(raw, 32, 64);
-            const float g = __shfl(gown, 16 * s + lc, 64) * dsoftplus20(raw + b2 + P.dbias);
+                for (int r = 0; r < 4; r++) raw = mfma16(w2p[t][r], fmaxf(h[t][r], 0.f), raw);
+            const float g = __shfl(gown, 16 * s + lc, 64) * dsoftplus20(raw[0] + P.dbias);
             if (lr == 0) ab2 += (double)g;
             f4 df[FT];
 #pragma unroll
@@ -1643,7 +1648,7 @@ __global__ __launch_bounds__(pf_bwd_threads(FM)) void prop_bwd_kernel(PropArgs P
     // the wavefronts' sums meet in LDS, one global atomic per weight and block
 #pragma unroll
     for (int t = 0; t < HT; t++) {
-        const int j = 16 * t + lc;
+        const int j = 16 * t + jl;
 #pragma unroll
         for (int q = 0; q < FT; q++)
 #pragma unroll
