@@ -1154,7 +1154,8 @@ constexpr int PF_HID = 64;
 constexpr int PF_MAXF = 32;
 constexpr int PF_FWD_THREADS = 256;
 // Adjoint: one block per CU while its registers allow 12 wavefronts (512 us at 4.2 M points and
-// 10 features; without the density's products 450, and 606 with three blocks of four; a third of the atomic additions at the end), else three.
+// 10 features; without the density's products 450, and 606 with three blocks of four; a third
+// of the atomic additions at the end), else three.
 constexpr int pf_bwd_threads(int fm) { return fm <= 12 ? 768 : 256; }
 
 struct PropArgs {
