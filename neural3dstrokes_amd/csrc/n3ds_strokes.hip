@@ -288,8 +288,10 @@ __global__ __launch_bounds__(BLOCK) void stroke_fwd_curve_kernel(
         for (int p = 0; p < np; p++) {
             const V3 xp = ld3(x + 3 * (nb + p));
             const V3 d = vmax0(vabs(xp - c) - h);
-            const float m = (reach + delta * radius[nb + p]) * 1.0001f + pad;
-            const bool far = dot(d, d) > m * m && 0.f * (xp.x + xp.y + xp.z) == 0.f;  // (a finite point)
+            const float r = radius[nb + p];
+            const float m = (reach + delta * r) * 1.0001f + pad;
+            // (a finite point; with a radius that is not positive, alpha may be one far away)
+            const bool far = dot(d, d) > m * m && 0.f * (xp.x + xp.y + xp.z) == 0.f && r > 0.f;
             const bool near = odd || !far;
             sal[wave][p][lane] = 0.f;
             qn = queue_push(q, qn, near && kv, (uint32_t)(p << 6 | lane));
