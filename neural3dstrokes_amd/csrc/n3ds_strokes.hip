@@ -329,10 +329,12 @@ __global__ __launch_bounds__(BLOCK) void stroke_fwd_curve_kernel(
 // the SDF: a hundredth of them.  Every pair's upstream is read once, lane per stroke, for
 // the colour sums; the live ones are queued and differentiated in full wavefronts, their
 // strokes' frames read from LDS, and summed per stroke in LDS as doubles (64-bit LDS float
-// atomics run 6 times as fast as 32-bit ones on this card).  The lane-per-stroke kernel
-// above runs the SDF's adjoint for 64 strokes as soon as one is live: 791 us at 65536
-// points x 500 cubic curves and 547 us at 262144 x 200 boxes; this one is bound by the 20
-// bytes read per pair.
+// atomics run 6 times as fast as 32-bit ones on this card).  What is not finite in a
+// stroke, a point or an upstream gradient reaches the gradients through any pair, as a
+// product with zero is then NaN: such a stroke's or point's pairs are all differentiated.
+// Looking for them once per block costs 1 us.  The lane-per-stroke kernel above runs the
+// SDF's adjoint for 64 strokes as soon as one is live: 791 us at 65536 points x 500 cubic
+// curves and 547 us at 262144 x 200 boxes; this one is bound by the 20 bytes read per pair.
 constexpr int LWAVES = 8;
 constexpr int LUNROLL = 4;  // points in flight per wavefront
 
@@ -350,13 +352,17 @@ __global__ __launch_bounds__(64 * LWAVES) __attribute__((amdgpu_waves_per_eu(4, 
     __shared__ float frame[64][NF + 1 - NF % 2];
     __shared__ double acc[NR][64];
     __shared__ double csum[NQ][64];
+    __shared__ int odd_stroke[64];
     __shared__ uint2 sq[LWAVES][128];  // point of the block << 6 | lane, dL/dalpha
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform per wavefront
     const int64_t k = (int64_t)blockIdx.y * 64 + lane;
     const bool kv = k < S;
     const int64_t kk = kv ? k : S - 1;
+    const int64_t n0 = (int64_t)blockIdx.x * ppb, n1 = min(N, n0 + ppb);
+    bool bad = false;
     if (wave == 0) {
         const float* row = sp + kk * P;
+        float zero = 0.f;  // NaN with a parameter that is not finite
         if (!is_curve(BASE)) {
             const Frame F = load_frame(row, P, flags);
 #pragma unroll
@@ -364,9 +370,26 @@ __global__ __launch_bounds__(64 * LWAVES) __attribute__((amdgpu_waves_per_eu(4, 
             frame[lane][9] = F.trans.x; frame[lane][10] = F.trans.y; frame[lane][11] = F.trans.z;
             frame[lane][12] = F.scale.x; frame[lane][13] = F.scale.y; frame[lane][14] = F.scale.z;
             frame[lane][15] = F.sz; frame[lane][16] = F.cz;
+            // (a point is divided by the scale)
+            zero = 0.f * (F.trans.x + F.trans.y + F.trans.z + F.scale.x + F.scale.y + F.scale.z) +
+                   0.f * (F.angle.x + F.angle.y + F.angle.z) + (0.f / F.scale.x + 0.f / F.scale.y + 0.f / F.scale.z);
         }
 #pragma unroll
-        for (int i = 0; i < NB; i++) frame[lane][FO + i] = row[i];
+        for (int i = 0; i < NB; i++) {
+            frame[lane][FO + i] = row[i];
+            zero += 0.f * row[i];
+        }
+        odd_stroke[lane] = !(zero == 0.f);
+    } else {
+        // (a radius of 0: the adjoint of the radius scale is infinite)
+        float zero = 0.f, least = INFINITY;
+        for (int64_t n = n0 + threadIdx.x - 64; n < n1; n += 64 * (LWAVES - 1)) {
+            const V3 xp = ld3(x + 3 * n);
+            const float r = radius[n];
+            zero += 0.f * (xp.x + xp.y + xp.z + r);
+            least = fminf(least, fabsf(r));
+        }
+        bad = !(zero == 0.f && least > 0.f);
     }
     for (int i = threadIdx.x; i < NR * 64; i += 64 * LWAVES) (&acc[0][0])[i] = 0.0;
     for (int i = threadIdx.x; i < NQ * 64; i += 64 * LWAVES) (&csum[0][0])[i] = 0.0;
@@ -376,8 +399,8 @@ __global__ __launch_bounds__(64 * LWAVES) __attribute__((amdgpu_waves_per_eu(4, 
         col[i] = cp[kk * Q + i];
         gc[i] = 0.f;
     }
-    __syncthreads();
-    const int64_t n0 = (int64_t)blockIdx.x * ppb, n1 = min(N, n0 + ppb);
+    const bool odd_points = __syncthreads_or(bad) != 0;  // some of the block's
+    const bool odd = odd_stroke[lane] != 0;
     uint2* q = sq[wave];
     int qn = 0;
     auto adjoint = [&](int i) {  // queue entry i of this lane
@@ -459,8 +482,13 @@ __global__ __launch_bounds__(64 * LWAVES) __attribute__((amdgpu_waves_per_eu(4, 
             if (nb + u >= n1) break;
             const V3 dir = (CID >= 2) ? ld3(viewdir + 3 * ((nb + u) / spr)) : v3s(0.f);
             color_grad_t<CID>(v3s(0.f), dir, col, gcv[u], gc, exact != 0);
-            // (an infinite or NaN upstream reaches the parameters through any pair)
-            const bool live = (0.f < al[u] && al[u] < 0.9999f) || !isfinite(ga[u]);
+            bool live = (0.f < al[u] && al[u] < 0.9999f) || !isfinite(ga[u]) || odd;
+            if (odd_points) {
+                const V3 xp = ld3(x + 3 * (nb + u));
+                const float r = radius[nb + u];
+                live = live || !(0.f * (xp.x + xp.y + xp.z + r) == 0.f) || r == 0.f;
+            }
+            live = live && kv;
             if (__ballot(live) == 0ull) continue;
             qn = queue_push(q, qn, live, make_uint2((uint32_t)((nb + u - n0) << 6 | lane), __float_as_uint(ga[u])));
             if (qn >= 64) {
