@@ -172,8 +172,12 @@ __global__ __launch_bounds__(64 * CWAVES) void compose_bwd_kernel(
             for (int c = 0; c < D; c++) ck[c] = v ? crow[k * D + c] : 0.f;
             const float Tin = G == 1 ? t_in[wave][ch] : t_grp[wave][ch % G];
             // without a nonzero alpha the chunk is transparent: everything behind a stroke is
-            // what lies behind the chunk, and the carry stays as it is
-            const bool clear = __ballot(a != 0.f) == 0ull;
+            // what lies behind the chunk, and the carry stays as it is (an infinite or NaN
+            // colour or density, whose product with an alpha of zero is NaN, goes the long way)
+            float zero = 0.f * dk;
+#pragma unroll
+            for (int c = 0; c < D; c++) zero += 0.f * ck[c];
+            const bool clear = __ballot(a != 0.f || !(zero == 0.f)) == 0ull;
             float Tk = Tin, Ubd = Ud, Rbk = Rb, Ubc[D];
 #pragma unroll
             for (int c = 0; c < D; c++) Ubc[c] = Uc[c];

@@ -63,3 +63,39 @@ def test_live_adjoint_passes_odd_values(base, kind, dev):
                     fin = torch.isfinite(b)
                     assert torch.equal(torch.isfinite(a), fin)
                     assert rel_err(a[fin], b[fin]) < (1e-4 if base in CURVES else 1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('value', [NAN, INF])
+@pytest.mark.parametrize('D', [1, 3])
+def test_compositing_passes_odd_values(D, value, dev):
+    """A transparent stroke with an infinite or NaN colour or density: alpha's gradients of the
+    strokes in front of it are not finite, whether or not a chunk of 64 holds another alpha
+    (one of 1e-30, which leaves every transmittance as it is)."""
+    g = torch.Generator().manual_seed(D)
+    N, S = 6, 256  # the chunks are strokes 192..255, 128..191, ...
+    a = torch.zeros(N, S)
+    a[:, [3, 70, 200]] = torch.rand(N, 3, generator=g) * 0.9
+    c, dp = torch.rand(N, S, D, generator=g), torch.rand(S, generator=g)
+    gd, gc = torch.randn(N, generator=g).to(dev), torch.randn(N, D, generator=g).to(dev)
+    out = []
+    for where in ('none', 'colour', 'density'):
+        cc, dd = c.clone(), dp.clone()
+        if where == 'colour':
+            cc[2, 150, D - 1] = value
+        elif where == 'density':
+            dd[140] = value
+        for tiny in (0.0, 1e-30):
+            at = a.clone()
+            at[:, 130] = tiny
+            t = [v.to(dev) for v in (at, cc, dd)]
+            for mode in ('exact', 'reference'):
+                ga, gcol, gdp = torch.full((N, S), 9.0, device=dev), torch.zeros_like(t[1]), torch.zeros_like(t[2])
+                backend.compose_backward(ga, gcol, gdp, gd, gc, *t, mode)
+                out.append((where, tiny, ga.cpu()))
+    for i in range(0, len(out), 4):
+        for (where, _, x), (_, _, y) in zip(out[i:i + 2], out[i + 2:i + 4]):
+            fin = torch.isfinite(y)
+            assert torch.equal(torch.isfinite(x), fin) and rel_err(x[fin], y[fin]) < 1e-5
+            assert bool(fin.all()) == (where == 'none')
+            assert where == 'none' or not fin[2, 200]
