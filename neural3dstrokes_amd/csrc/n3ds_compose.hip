@@ -161,6 +161,7 @@ __global__ __launch_bounds__(64 * CWAVES) void compose_bwd_kernel(
                     if (lane == 0) t_grp[wave][c2 - g0] = Tg;
                     Tg = __shfl(Tg * scan_prod_excl(f2, lane) * f2, 63, 64);
                 }
+                wave_fence();  // t_grp is read by every lane
             }
             int64_t k = S - 1 - ((int64_t)ch * 64 + lane);
             bool v = k >= 0;

@@ -1615,6 +1615,7 @@ __global__ __launch_bounds__(pf_bwd_threads(FM)) void prop_bwd_kernel(PropArgs P
             for (int q = 0; q < FT; q++)
 #pragma unroll
                 for (int r = 0; r < 4; r++) ft[q][r] = pt[16 * s + 4 * lr + r][16 * q + lc];
+            wave_fence();  // every lane has read the rows that the gradients go to below
             f4 h[HT];
 #pragma unroll
             for (int t = 0; t < HT; t++) {
