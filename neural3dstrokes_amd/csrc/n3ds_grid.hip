@@ -1153,14 +1153,18 @@ static int gs_launch(const T* grad, const float* inputs, const int* offsets, int
 constexpr int PF_HID = 64;
 constexpr int PF_MAXF = 32;
 constexpr int PF_FWD_THREADS = 256;
-// Adjoint: one block per CU while its registers allow 12 wavefronts (512 us at 4.2 M points and
-// 10 features; without the density's products 450, and 606 with three blocks of four; a third
-// of the atomic additions at the end), else three.
+// Adjoint: persistent blocks, as many as a CU holds at once.  Up to 12 features one block of 12
+// wavefronts (512 us at 4.2 M points and 10 features; without the density's products 450, and
+// 606 with three blocks of four; a third of the atomic additions at the end), beyond them blocks
+// of 4: two up to 20 features, one above, where a wavefront needs more than 256 registers.  (Three
+// blocks launched where two or one fit: 897 instead of 750 us at 16 features, 1500 instead of
+// 921 at 20, 1930 instead of 1880 at 28, with the torch calls around them.)
 constexpr int pf_bwd_threads(int fm) { return fm <= 12 ? 768 : 256; }
+constexpr int pf_bwd_blocks(int fm) { return fm > 12 && fm <= 20 ? 2 : 1; }
 // Tiles of 64 points whose weight gradients a wavefront sums in float32 before they go to the
 // block's doubles.  With all of its points in one chain, dW1 of 2^24 equal points was off by
-// 5.0e-5 of its largest entry, now 2.7e-6; the backward takes 646 -> 610 us at 2^20 points and
-// 10 features, 2 to 8 % more at 20.
+// 5.0e-5 of its largest entry, now 2.7e-6, in no more time at 10 features (570 us at 4.2 M
+// points with the torch calls around it) and 3 % more at 28.
 constexpr int PF_HELD = 4;
 
 struct PropArgs {
@@ -1511,7 +1515,7 @@ __device__ __forceinline__ f4 mfma16(float a, float b, f4 c) {
 // 72 matrix instructions per 16 points and 10 features.  The vector version went through
 // LDS for every product (7 LDS reads per point and hidden unit): 1560 us at 4.2 M points.
 template <typename T, int C, int FM, int FX = 0>
-__global__ __launch_bounds__(pf_bwd_threads(FM)) void prop_bwd_kernel(PropArgs P, const float* __restrict__ gdens,
+__global__ __launch_bounds__(pf_bwd_threads(FM), pf_bwd_blocks(FM)) void prop_bwd_kernel(PropArgs P, const float* __restrict__ gdens,
                                                                   const float* __restrict__ feat_in,
                                                                   float* __restrict__ gfeat, float* __restrict__ x01_out,
                                                                   float* __restrict__ gW1, float* __restrict__ gb1,
@@ -2036,7 +2040,7 @@ static int prop_field_backward(double* gsum, const float* coords, int64_t n_poin
     int64_t nb;
     hipStream_t s = (hipStream_t)stream;
 #define LAUNCH_PB(CC, FM, FX)                                                                                    \
-    st = prop_blocks(n_points, pf_bwd_threads(FM), 768 / pf_bwd_threads(FM), &nb);                              \
+    st = prop_blocks(n_points, pf_bwd_threads(FM), pf_bwd_blocks(FM), &nb);                                      \
     if (st) return st;                                                                                          \
     if (dtype == 0)                                                                                              \
         hipLaunchKernelGGL((prop_bwd_kernel<float, CC, FM, FX>), dim3((unsigned)nb), dim3(pf_bwd_threads(FM)), 0, s, \
