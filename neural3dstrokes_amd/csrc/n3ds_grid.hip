@@ -1227,8 +1227,8 @@ __device__ __forceinline__ void prop_features(const PropArgs& P, const float* x0
 // the L2 are then bound by the vector cache, 2 to 3 clocks a line: a load of 16 bytes serves
 // both corners of most x edges.  The rows of a point's corners wait in registers until the last
 // part, so that they are summed in the one kernel's order, to the bit (a hidden unit at its
-// kink passes on or not by the last bit of its features).  Features are written level by
-// level, [L, n, C]; with the head after it 1435 us (1538 + 140 with whole levels of 8 MB, 1149 +
+// kink passes on or not by the last bit of its features); two features a row do not fit the
+// registers that way and take a level whole.  Features are written level by level, [L, n, C]; with the head after it 1435 us (1538 + 140 with whole levels of 8 MB, 1149 +
 // 140 with sums kept from part to part).
 constexpr int LS_THREADS = 1024;
 constexpr int LS_POINTS = 8;                // per thread and round at most
@@ -1381,7 +1381,7 @@ __global__ __launch_bounds__(LS_THREADS) void prop_level_kernel(PropArgs P, int6
             const bool hashed = !P.align && P.gridtype == 0 && r1 < 65536u && !lattice && (hs & (hs - 1)) == 0 &&
                                 !(r1 >= 1626u && r1 * r1 <= hs) && hs >= 16 && ((uintptr_t)g & 15) == 0;
             const uint32_t part = (uint32_t)(LS_PART_BYTES / (C * (int)sizeof(T)));
-            if (hashed && hs > part) {
+            if (C == 1 && hashed && hs > part) {
                 GridRow<T, C> row[LS_POINTS][8];
 #pragma unroll
                 for (int q = 0; q < LS_POINTS; q++)
@@ -1918,8 +1918,9 @@ static PropArgs prop_args(const float* coords, int64_t N, int warp, float box_si
 // features, staged against fused (us), 10 levels:
 //   rows of 4 bytes, tables of 57 MB: 2^17 points 75 / 65, 2^18 97 / 122, 2^22 1435 / 1848;
 //   15 MB: 2^17 65 / 47, 2^18 72 / 88, 2^22 970 / 1420; 4.2 MB: 2^18 62 / 63, 2^21 385 / 437;
-//   two half features, levels of 2 MB: 2^17 73 / 50, 2^18 89 / 93, 2^22 1130 / 1478; of 8 MB:
-//   2^18 244 / 126, 2^21 1092 / 930;
+//   two half features, levels of 2 MB: 2^17 73 / 50, 2^18 89 / 93, 2^22 1130 / 1478; four of
+//   ten of 8 MB (42 MB; the whole call): 2^20 640 / 610, 2^22 1863 / 1870 (in parts, spilling the
+//   rows kept: 750, 2185);
 //   rows of 8 bytes, 30 MB: 2^18 117 / 110, 2^21 917 / 862; of 16 bytes: 2^21 1412 / 1119.
 constexpr int64_t PF_STAGE_TABLE = 4 << 20;  // bytes of all tables
 constexpr int64_t PF_STAGE_ROW = 4;          // bytes of a row at most
@@ -1931,7 +1932,7 @@ N3DS_EXPORT int64_t n3ds_prop_field_workspace_bytes(int64_t n_points, int num_le
     if (n_points < PF_STAGE_POINTS || num_levels < 1 || level_dim < 1 || n_rows < 0) return 0;
     const int64_t row = level_dim * (dtype == 1 ? 2 : 4);
     if (row > PF_STAGE_ROW || n_rows * row <= PF_STAGE_TABLE) return 0;
-    // two half features in parts of a level: the rows kept do not fit the registers
+    // two half features take a level whole: past an L2 a level on average the gathers leave it
     if (level_dim == 2 && n_rows * row > num_levels * LS_PART_BYTES) return 0;
     return std::min(n_points, PF_STAGE_CHUNK) * num_levels * level_dim * 4;
 }
