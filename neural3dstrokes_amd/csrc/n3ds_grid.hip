@@ -1922,16 +1922,29 @@ static PropArgs prop_args(const float* coords, int64_t N, int warp, float box_si
 //   ten of 8 MB (42 MB; the whole call): 2^20 640 / 610, 2^22 1863 / 1870 (in parts, spilling the
 //   rows kept: 750, 2185);
 //   rows of 8 bytes, 30 MB: 2^18 117 / 110, 2^21 917 / 862; of 16 bytes: 2^21 1412 / 1119.
+// The head of ten levels is compiled for its 10 or 20 features; any other count's loops to 16 or
+// 32, which the one kernel does in the shadow of its gathers, so there levels must stay in an L2
+// (2 MB at most) for more points (the whole call, 2^20 and 2^22 points):
+//   7 levels to 2 MB: 394 / 383, 1201 / 1185; 8: 438 / 443, 1386 / 1427; 16: 866 / 942, 2934 / 3412;
+//   8 levels to 4 MB: 520 / 489, 1690 / 1583; 16: 1121 / 1016, 3400 / 3400; to 8 MB: 551 / 539,
+//   1763 / 1726; 1154 / 1109, 3685 / 3876; two half features, 12 levels to 4 MB: 1026 / 900,
+//   3304 / 3001.
 constexpr int64_t PF_STAGE_TABLE = 4 << 20;  // bytes of all tables
 constexpr int64_t PF_STAGE_ROW = 4;          // bytes of a row at most
 constexpr int64_t PF_STAGE_POINTS = 1 << 18;
 constexpr int64_t PF_STAGE_CHUNK = 1 << 22;  // points whose features are staged at one time
+constexpr int PF_STAGE_LEVELS = 8;               // not ten of them: levels,
+constexpr int64_t PF_STAGE_LEVEL = 7 << 18;      // bytes of one on average at most,
+constexpr int64_t PF_STAGE_MORE = 1 << 20;       // and points
 
 N3DS_EXPORT int64_t n3ds_prop_field_workspace_bytes(int64_t n_points, int num_levels, int level_dim, int64_t n_rows,
                                                     int dtype) {
     if (n_points < PF_STAGE_POINTS || num_levels < 1 || level_dim < 1 || n_rows < 0) return 0;
     const int64_t row = level_dim * (dtype == 1 ? 2 : 4);
     if (row > PF_STAGE_ROW || n_rows * row <= PF_STAGE_TABLE) return 0;
+    if (num_levels != 10 && (level_dim != 1 || num_levels < PF_STAGE_LEVELS || n_points < PF_STAGE_MORE ||
+                             n_rows * row > num_levels * PF_STAGE_LEVEL))
+        return 0;
     // two half features take a level whole: past an L2 a level on average the gathers leave it
     if (level_dim == 2 && n_rows * row > num_levels * LS_PART_BYTES) return 0;
     return std::min(n_points, PF_STAGE_CHUNK) * num_levels * level_dim * 4;
