@@ -1463,7 +1463,7 @@ __global__ __launch_bounds__(PF_FWD_THREADS) void prop_fwd_kernel(PropArgs P, co
     const float b2 = P.b2[0];
     for (int64_t i = (int64_t)blockIdx.x * PF_FWD_THREADS + threadIdx.x; i < n;
          i += (int64_t)gridDim.x * PF_FWD_THREADS) {
-        const int64_t b = b0 + i;
+        const int64_t b = STAGED ? b0 + i : i;  // (b0 is 0 without the stage)
         float cw[3], x01[3], f[FM];
         prop_warp(P, b, cw, x01);
         if constexpr (STAGED) {
