@@ -56,7 +56,9 @@ __device__ __forceinline__ float sf_cdf(float* cw, int j, int m, float v, float 
 
 // NB > 0: at most 64 NB bins, their logits and exponentials in registers (0: any number, read
 // and exponentiated again for each use): 67 instead of 75 us at 65536 rays, 192 bins and 128
-// samples, with the two searches of a lane side by side.
+// samples, with the two searches of a lane side by side.  (A second search that no sample of the
+// last 64 needs cost 73 instead of 63 us at 65 bins and 64 samples, and side by side past 256
+// bins 130 instead of 120 at 300 bins and 128 samples.)
 template <int NB>
 __global__ __launch_bounds__(256) void sample_intervals_kernel(float* __restrict__ t_out,
                                                                const float* __restrict__ t,
@@ -115,13 +117,14 @@ __global__ __launch_bounds__(256) void sample_intervals_kernel(float* __restrict
         sf_wave_sync();
         float* outr = t_out + r * (n + 1);
         const float* jr = jitter ? jitter + r * jitter_width : nullptr;
-        for (int i = lane; i < n; i += 128) {  // two searches side by side
-            const int i1 = i + 64 < n ? i + 64 : i;
-            float u0 = u_base[i], u1 = u_base[i1];
-            if (jr) {
-                u0 = __fadd_rn(u0, __fmul_rn(jr[jitter_width == 1 ? 0 : i], max_jitter));
-                u1 = __fadd_rn(u1, __fmul_rn(jr[jitter_width == 1 ? 0 : i1], max_jitter));
-            }
+        auto position = [&](int i) {
+            const float u = u_base[i];
+            return jr ? __fadd_rn(u, __fmul_rn(jr[jitter_width == 1 ? 0 : i], max_jitter)) : u;
+        };
+        int i0 = 0;
+        for (; NB > 0 && i0 + 64 < n; i0 += 128) {  // two searches side by side
+            const int i = i0 + lane, i1 = min(i + 64, n - 1);
+            const float u0 = position(i), u1 = position(i1);
             int lo0 = 0, hi0 = m + 1, lo1 = 0, hi1 = m + 1;  // first index with cw[idx] > u
             for (int left = m + 1; left > 0; left >>= 1) {
                 const int mid0 = (lo0 + hi0) >> 1, mid1 = (lo1 + hi1) >> 1;
@@ -134,6 +137,16 @@ __global__ __launch_bounds__(256) void sample_intervals_kernel(float* __restrict
             }
             cs[i] = sf_center(cw, te, m, u0, lo0);
             if (i + 64 < n) cs[i1] = sf_center(cw, te, m, u1, lo1);
+        }
+        for (int i = i0 + lane; i < n; i += 64) {  // at most 64 are left
+            const float u = position(i);
+            int lo = 0, hi = m + 1;
+            while (lo < hi) {
+                const int mid = (lo + hi) >> 1;
+                if (cw[mid] <= u) lo = mid + 1;
+                else hi = mid;
+            }
+            cs[i] = sf_center(cw, te, m, u, lo);
         }
         sf_wave_sync();
         for (int o = lane; o <= n; o += 64) {
