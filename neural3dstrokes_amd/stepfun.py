@@ -18,9 +18,11 @@ from . import _lib
 def resample_logits(sdist, weights, resample_padding=0.0):
     """models.py:168-171: log(w + padding) on bins of positive width, -inf elsewhere."""
     # three elementwise passes instead of five: log of -0 and of 0 are the same, and -inf needs
-    # no tensor of its own where it does not decide the result's type
-    padded = weights if isinstance(resample_padding, (int, float)) and resample_padding == 0 else \
-        weights + resample_padding
+    # no tensor of its own where it does not decide the result's type.  The logarithm of weights
+    # with gradients keeps its argument, which is then not the caller's own tensor: that one may
+    # be changed before the backward, and a weight of -0 has 1 / 0 as its slope, not 1 / -0.
+    plain = isinstance(resample_padding, (int, float)) and resample_padding == 0 and not weights.requires_grad
+    padded = weights if plain else weights + resample_padding
     logits = torch.log(padded)
     empty = -torch.inf if logits.dtype == sdist.dtype else torch.full_like(sdist[..., :-1], -torch.inf)
     return torch.where(sdist[..., 1:] > sdist[..., :-1], logits, empty)
