@@ -65,7 +65,9 @@ def _check_device_ids(stroke_ids, Pmax, status):
 # recomputation chunk by chunk.  Capacities per ray: hits min(S, 2n), pairs 8n.
 # The Laplace transfer's tail reaches several stroke widths (7 to 12 n live pairs
 # per ray were counted on fields of 150 to 300 solids, 0.2 to 0.4 n with the linear
-# transfer), so it keeps 8n hits and 32n pairs where those fit the budget.
+# transfer), so it keeps 8n hits and 32n pairs where those fit the budget, and the backward's
+# workspace has room for 16n more adjoint records (32 B) per ray in what is left of it; where
+# the memory does not hold either, both are as for the linear transfer.
 STORE_BUDGET_BYTES = 8 << 30
 
 
@@ -78,28 +80,47 @@ def keep_capacities(R, n, S, color_id, wide=False):
     return cap_h, cap_p, npf, nch, nbytes
 
 
-def _split_records(R, n, laplace):
+def _split_records(R, n, laplace, cap_p, kept_bytes):
     """Floats of adjoint records beyond the library's default to make room for in the
-    backward's workspace: 16n live pairs of 8 floats per ray with the Laplace transfer,
-    up to half of the kept activations' budget."""
-    return min(R * n * 16 * 8, STORE_BUDGET_BYTES // 8) if laplace else 0
+    backward's workspace: 16n live pairs of 8 floats per ray with the Laplace transfer, no
+    more than were kept, within what the kept activations leave of their budget."""
+    if not laplace:
+        return 0
+    return min(R * min(16 * n, cap_p) * 8, max(0, STORE_BUDGET_BYTES - kept_bytes) // 4)
 
 
 def _keep_buffers(store, R, n, S, color_id, laplace, dev):
     if store is False:
         return None
+    npf, nch = (4 if color_id == 1 else 1), (S + 63) // 64
     if isinstance(store, tuple):
-        cap_h, cap_p = store
-        npf, nch = (4 if color_id == 1 else 1), (S + 63) // 64
+        caps = [store]
     else:
-        cap_h, cap_p, npf, nch, nbytes = keep_capacities(R, n, S, color_id, laplace)
-        if laplace and nbytes > STORE_BUDGET_BYTES:
-            cap_h, cap_p, npf, nch, nbytes = keep_capacities(R, n, S, color_id)
-        if store == 'auto' and nbytes > STORE_BUDGET_BYTES:
+        caps = [keep_capacities(R, n, S, color_id)]
+        if store == 'auto' and caps[0][4] > STORE_BUDGET_BYTES:
             return None
-    return (torch.empty(R * nch * 3, dtype=torch.int32, device=dev),
-            torch.empty(R * cap_h * 4, dtype=torch.int32, device=dev),
-            torch.empty(R * npf * cap_p, dtype=torch.float32, device=dev), cap_h, cap_p)
+        if laplace:
+            wide = keep_capacities(R, n, S, color_id, True)
+            if wide[4] <= STORE_BUDGET_BYTES:
+                caps.insert(0, wide)
+    for i, (cap_h, cap_p) in enumerate(c[:2] for c in caps):
+        try:
+            return (torch.empty(R * nch * 3, dtype=torch.int32, device=dev),
+                    torch.empty(R * cap_h * 4, dtype=torch.int32, device=dev),
+                    torch.empty(R * npf * cap_p, dtype=torch.float32, device=dev), cap_h, cap_p)
+        except torch.cuda.OutOfMemoryError:  # the wider buffers are for speed only
+            if i == len(caps) - 1:
+                raise
+
+
+def _workspace(floats, extra, dev):
+    """floats + extra of scratch, or floats where that does not fit the memory."""
+    if extra > 0:
+        try:
+            return torch.empty(floats + extra, dtype=torch.float32, device=dev)
+        except torch.cuda.OutOfMemoryError:
+            pass
+    return torch.empty(max(floats, 1), dtype=torch.float32, device=dev)
 
 
 def _launch_forward(origins, directions, viewdirs, radii, tdist, stroke_ids, shape_params, color_params,
@@ -192,11 +213,15 @@ class _render_fn(Function):
         g_rgb = torch.zeros(R, 3, device=dev) if g_rgb is None else g_rgb.float().contiguous()
         g_acc = None if g_acc is None else g_acc.float().contiguous()
         g_depth = None if g_depth is None else g_depth.float().contiguous()
+        records = 0
         if scenes is None:
             nws = _lib.lib().n3ds_render_backward_workspace_floats(R, S, Pmax, Q)
             if hd.numel() > 0 and nws >= 0:  # kept hits: room for the split adjoint
                 nsp = _lib.lib().n3ds_render_backward_split_floats(R, S, Pmax, Q)
-                nws = -1 if nsp < 0 else max(nws, nsp + (_split_records(R, n1 - 1, laplace) if nsp else 0))
+                nws = -1 if nsp < 0 else max(nws, nsp)
+                if nsp > 0:  # and for more records than its default where many pairs are live
+                    kept = 4 * (hd.numel() + hb.numel() + pb.numel())
+                    records = max(0, nsp + _split_records(R, n1 - 1, laplace, cap_p, kept) - nws)
             bwd, batch_args = _lib.lib().n3ds_render_backward, ()
         else:
             nws = _lib.lib().n3ds_render_batch_backward_workspace_floats(scenes.host_ptr(), scenes.n_scenes, n1 - 1,
@@ -204,7 +229,7 @@ class _render_fn(Function):
             bwd, batch_args = _lib.lib().n3ds_render_batch_backward, scenes.c_args()
         if nws < 0:
             _lib.check(2)
-        ws = torch.empty(max(int(nws), 1), dtype=torch.float32, device=dev)
+        ws = _workspace(int(nws), records, dev)
         gs = torch.zeros_like(shape_params)
         gc = torch.zeros_like(color_params)
         gd = torch.zeros_like(density_params)
