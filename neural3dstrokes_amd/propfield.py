@@ -49,7 +49,12 @@ class _prop_field_fn(Function):
         x01 = torch.empty(N, 3, dtype=torch.float32, device=dev) if keep else None
         rows, flag = embeddings.shape[0], _grid._dtype_flag(embeddings)
         nws = int(_lib.lib().n3ds_prop_field_workspace_bytes(N, L, C, rows, flag))
-        ws = torch.empty(nws, dtype=torch.uint8, device=dev) if nws > 0 else None
+        ws = None
+        if nws > 0:
+            try:
+                ws = torch.empty(nws, dtype=torch.uint8, device=dev)
+            except torch.cuda.OutOfMemoryError:  # one kernel does without
+                nws = 0
         _lib.check(_lib.lib().n3ds_prop_field_forward_ws(
             _lib.ptr(coords), N, warp, float(box), _lib.ptr(embeddings), _lib.ptr(offsets), L, C, S, H, gridtype,
             align, interp, flag, _lib.ptr(w1), _lib.ptr(b1), _lib.ptr(w2), _lib.ptr(b2), float(dbias),
