@@ -768,9 +768,13 @@ static GsWs gs_carve(void* ws, int64_t B, int C, int L) {
 }
 
 // Lattices wider than a bucket do not fit (their x moves the row out of it), and past 256
-// buckets per level the tiles' segments get much shorter than a wavefront.
+// buckets per level the tiles' segments get much shorter than a wavefront.  Few points do not
+// fill the tiles of a block per CU (16 levels of up to 2^19 rows, sorted against bucketed in us:
+// 1 feature 256 points 35 / 38, 16 28 / 27; 2 features 1024 points 61 / 76, 256 43 / 38; 4 features
+// 4096 points 110 / 231, 1024 93 / 88).
 static bool gs_applies(int64_t B, int D, int C, int L, int64_t n_rows, int gridtype, int align, const LevelTab& lt) {
     if (D != 3 || gridtype != 0 || align || B >= (1ll << 28) || n_rows > (int64_t)256 * L * gs_rows(C)) return false;
+    if (B < (C < 4 ? 512 * C : 2048)) return false;
     for (int l = 0; l < L; l++)
         if (!(lt.scale[l] + 3.f < (float)gs_rows(C))) return false;
     return true;
