@@ -3598,6 +3598,15 @@ N3DS_EXPORT int n3ds_render_forward(const float* origins, const float* direction
 // with their group counts (as many as the workspace given holds, at least min_pages).
 constexpr int SPLIT_WAVES = 4;
 
+// With rows of floats that nearly fill the LDS there are strokes enough for many rays to hit more
+// than are kept, and those run in the fused kernel after the others: the split then pays only for
+// many rays and, with wide rows, not too many strokes.  Split against fused, us, 64 samples:
+// 2000 strokes x 18 columns 594 / 467 at 4096 rays, 1103 / 1008 at 16384, 2739 / 2810 at 65536;
+// 2150 x 18 648 / 537, 1185 / 1070, 2964 / 2893; 1400 x 27 400 / 316, 555 / 578, 1209 / 1644; 1500
+// x 27 406 / 341, 679 / 683, 1302 / 1683.
+constexpr int64_t SPLIT_FULL_RAYS = 16384;
+constexpr int SPLIT_FULL_STROKES = 1536;
+
 typedef void (*PairsKernel)(RenderArgs, float*);
 
 struct SplitPlan {
@@ -3634,6 +3643,7 @@ static int split_plan(int ns, int cid, int64_t n_rays, int S, int PG, SplitPlan*
     const bool wide = (int64_t)S * PG * 8 <= g_max_lds;  // rows of doubles in the pair kernel
     sp->lds2 = (int64_t)S * PG * (wide ? 8 : 4);
     if (sp->lds2 > g_max_lds) return N3DS_OK;
+    if (sp->lds2 > g_max_lds / 8 * 7 && !wide && (n_rays < SPLIT_FULL_RAYS || S > SPLIT_FULL_STROKES)) return N3DS_OK;
     sp->k2 = pairs_kernel_ptr(cid, wide);
     sp->lds1 = (int64_t)SPLIT_WAVES * split_wave_floats(ns) * 4;
     sp->k1 = bwd_kernel_ptr(ns, cid, 2);
