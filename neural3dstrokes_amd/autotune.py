@@ -18,8 +18,8 @@ Tunes, by timing the real workload on the device, the parameters exposed by
 * ``bwd_split``: with the forward's kept hits, the adjoint runs as a per-ray
   kernel that lists its live pairs' adjoint records per SDF family and a kernel
   over those records (1), or as one kernel (0);
-* ``split_cap``: records per ray and family the split adjoint's lists hold (a
-  fuller list makes the one-kernel adjoint take every ray).
+* ``split_cap``: records per ray and family that the split adjoint's pool is
+  sized for (rays that find it empty are left to the one-kernel adjoint).
 
 Results do not depend on them beyond float summation order.  ``tune`` runs a
 caller-supplied step over a small grid (coordinate descent, one parameter at a

@@ -1198,8 +1198,8 @@ constexpr int PF_HID = 64;
 constexpr int PF_MAXF = 32;
 constexpr int PF_FWD_THREADS = 256;
 // Adjoint: persistent blocks, as many as a CU holds at once.  Up to 12 features one block of 12
-// wavefronts (512 us at 4.2 M points and 10 features; without the density's products 450, and
-// 606 with three blocks of four; a third of the atomic additions at the end), beyond them blocks
+// wavefronts (522 us at 4.2 M points and 10 features; without the density's products, each with
+// one float32 chain a wavefront, 450 of 512, and 606 with three blocks of four), beyond them blocks
 // of 4: two up to 20 features, one above, where a wavefront needs more than 256 registers.  (Three
 // blocks launched where two or one fit: 897 instead of 750 us at 16 features, 1500 instead of
 // 921 at 20, 1930 instead of 1880 at 28, with the torch calls around them.)
@@ -1272,8 +1272,9 @@ __device__ __forceinline__ void prop_features(const PropArgs& P, const float* x0
 // both corners of most x edges.  The rows of a point's corners wait in registers until the last
 // part, so that they are summed in the one kernel's order, to the bit (a hidden unit at its
 // kink passes on or not by the last bit of its features); two features a row do not fit the
-// registers that way and take a level whole.  Features are written level by level, [L, n, C]; with the head after it 1435 us (1538 + 140 with whole levels of 8 MB, 1149 +
-// 140 with sums kept from part to part).
+// registers that way and take a level whole.  Features are written level by level, [L, n, C]; with
+// the head after it 1435 us (1538 + 140 with whole levels of 8 MB, 1149 + 140 with sums kept from
+// part to part).
 constexpr int LS_THREADS = 1024;
 constexpr int LS_POINTS = 8;                // per thread and round at most
 constexpr int64_t LS_PART_BYTES = 4 << 20;  // of a level's table gathered from at one time
@@ -1728,7 +1729,7 @@ __global__ __launch_bounds__(pf_bwd_threads(FM), pf_bwd_blocks(FM)) void prop_bw
     drain();
     if (lr == 0) atomicAdd(&sum[PF_HID * (FM + 2)], ab2);
     __syncthreads();
-    if (gsum) {  // [W1 | b1 | W2 | b2] in doubles: the order of the blocks leaves no rounding in them
+    if (gsum) {  // [W1 | b1 | W2 | b2] in doubles: what the order of the blocks rounds is far below a float's last bit
         for (int i = threadIdx.x; i < PF_HID * (F + 2) + 1; i += NT)
             atomicAdd(&gsum[i], i < PF_HID * F ? sum[(i / F) * FM + i % F] : sum[PF_HID * FM + i - PF_HID * F]);
         return;

@@ -2545,7 +2545,7 @@ __global__ __launch_bounds__(64 * BWAVES) void render_bwd_kernel(RenderArgs A0, 
     constexpr int NQ = num_color_params(CID);
     constexpr int NG = 15 + NQ;  // gradient slots per pair
     // live-pair codes (hit << 2 | class) and lists (hit << SH | pair); MODE 2 has them in 16
-    // bits and no gradient slots, which leaves room for four of its blocks on a CU instead of
+    // bits and no gradient slots, which leaves LDS for four of its blocks on a CU instead of
     // three (278 instead of 343 us on the 500-stroke palette, 65536 rays x 128 samples)
     typedef typename std::conditional<MODE == 2, short, int>::type Code;
     typedef typename std::conditional<MODE == 2, unsigned short, int>::type Live;
