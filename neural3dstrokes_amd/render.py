@@ -92,25 +92,27 @@ def _split_records(R, n, laplace, cap_p, kept_bytes):
 def _keep_buffers(store, R, n, S, color_id, laplace, dev):
     if store is False:
         return None
-    npf, nch = (4 if color_id == 1 else 1), (S + 63) // 64
     if isinstance(store, tuple):
-        caps = [store]
+        cap_h, cap_p = store
+        npf, nch = (4 if color_id == 1 else 1), (S + 63) // 64
     else:
-        caps = [keep_capacities(R, n, S, color_id)]
-        if store == 'auto' and caps[0][4] > STORE_BUDGET_BYTES:
+        cap_h, cap_p, npf, nch, nbytes = keep_capacities(R, n, S, color_id)
+        if store == 'auto' and nbytes > STORE_BUDGET_BYTES:
             return None
         if laplace:
             wide = keep_capacities(R, n, S, color_id, True)
             if wide[4] <= STORE_BUDGET_BYTES:
-                caps.insert(0, wide)
-    for i, (cap_h, cap_p) in enumerate(c[:2] for c in caps):
-        try:
-            return (torch.empty(R * nch * 3, dtype=torch.int32, device=dev),
-                    torch.empty(R * cap_h * 4, dtype=torch.int32, device=dev),
-                    torch.empty(R * npf * cap_p, dtype=torch.float32, device=dev), cap_h, cap_p)
-        except torch.cuda.OutOfMemoryError:  # the wider buffers are for speed only
-            if i == len(caps) - 1:
-                raise
+                try:
+                    return _kept(R, npf, nch, *wide[:2], dev)
+                except torch.cuda.OutOfMemoryError:  # the wider buffers are for speed only
+                    pass
+    return _kept(R, npf, nch, cap_h, cap_p, dev)
+
+
+def _kept(R, npf, nch, cap_h, cap_p, dev):
+    return (torch.empty(R * nch * 3, dtype=torch.int32, device=dev),
+            torch.empty(R * cap_h * 4, dtype=torch.int32, device=dev),
+            torch.empty(R * npf * cap_p, dtype=torch.float32, device=dev), cap_h, cap_p)
 
 
 def _workspace(floats, extra, dev):
@@ -219,7 +221,7 @@ class _render_fn(Function):
             if hd.numel() > 0 and nws >= 0:  # kept hits: room for the split adjoint
                 nsp = _lib.lib().n3ds_render_backward_split_floats(R, S, Pmax, Q)
                 nws = -1 if nsp < 0 else max(nws, nsp)
-                if nsp > 0:  # and for more records than its default where many pairs are live
+                if laplace and nsp > 0:  # and for more records than its default, as many pairs are live
                     kept = 4 * (hd.numel() + hb.numel() + pb.numel())
                     records = max(0, nsp + _split_records(R, n1 - 1, laplace, cap_p, kept) - nws)
             bwd, batch_args = _lib.lib().n3ds_render_backward, ()
