@@ -1672,13 +1672,16 @@ __global__ __launch_bounds__(pf_bwd_threads(FM), pf_bwd_blocks(FM)) void prop_bw
 #pragma unroll
                 for (int k = 0; k < KS; k++) h[t] = mfma16(w1[t][k], f[k], h[t]);
             }
+            // without a point in the last tile no unit is on and the gradient is 0, whatever the
+            // weights are (0 times an infinite one is NaN)
+            const bool on = 16 * s + lc < np;
             // every row of the product is the density's pre-activation, its 64 terms in order
             f4 raw = (f4){b2, b2, b2, b2};
 #pragma unroll
             for (int t = 0; t < HT; t++)
 #pragma unroll
                 for (int r = 0; r < 4; r++) raw = mfma16(w2p[t][r], fmaxf(h[t][r], 0.f), raw);
-            const float g = __shfl(gown, 16 * s + lc, 64) * dsoftplus20(raw[0] + P.dbias);
+            const float gp = __shfl(gown, 16 * s + lc, 64) * dsoftplus20(raw[0] + P.dbias), g = on ? gp : 0.f;
             if (lr == 0) ab2 += (double)g;
             f4 df[FT];
 #pragma unroll
@@ -1687,7 +1690,7 @@ __global__ __launch_bounds__(pf_bwd_threads(FM), pf_bwd_blocks(FM)) void prop_bw
             for (int t = 0; t < HT; t++)
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
-                    const float dh = h[t][r] > 0.f ? g * w2p[t][r] : 0.f;
+                    const float dh = h[t][r] > 0.f && on ? g * w2p[t][r] : 0.f;
 #pragma unroll
                     for (int q = 0; q < FT; q++) df[q] = mfma16(w1t[q][t][r], dh, df[q]);
                 }
@@ -1701,7 +1704,7 @@ __global__ __launch_bounds__(pf_bwd_threads(FM), pf_bwd_blocks(FM)) void prop_bw
                 for (int k = 0; k < KS; k++) hq = mfma16(f[k], w1[t][k], hq);
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
-                    const float dh = hq[r] > 0.f ? gq[r] * w2q[t] : 0.f;
+                    const float dh = hq[r] > 0.f && 16 * s + 4 * lr + r < np ? gq[r] * w2q[t] : 0.f;
                     ab1[t] += dh;
                     aw2[t] += gq[r] * fmaxf(hq[r], 0.f);
 #pragma unroll
